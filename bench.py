@@ -64,8 +64,8 @@ def algorithmic_work(x, y, p2, p3, owner, H2=16, W2=20):
     measurement's per-record accounting (each layer's input rows, the
     hidden-state read and write per pair, the output slots; weights excluded,
     they stay in cache) and the bytes each launch moves at its interface,
-    which also counts this design's intermediates (the projections' [v | g]
-    pair rows, the recurrence's h rows).  Returns ({phase: flops},
+    which also counts the intermediates of a drain in separate launches (the
+    projections' [v | g] pair rows, the recurrence's h rows).  Returns ({phase: flops},
     {phase: algorithmic bytes}, {phase: interface bytes}, total MACs)."""
     x = x.astype(np.int64)
     y = y.astype(np.int64)
@@ -115,9 +115,9 @@ def algorithmic_work(x, y, p2, p3, owner, H2=16, W2=20):
     }
     # the recurrence h = sigmoid(g) h + v over every pair entering the layer
     # (sigmoid ~ 4 FLOP, the map composition and the replay 2 FMA):
-    # algorithmically the pair's hidden state is read and written; one launch
-    # (k_scan, in the apply slot) reads each pair's v, g rows once and writes
-    # h where the output is consumed
+    # algorithmically the pair's hidden state is read and written; it takes
+    # each pair's v, g rows from the projection and writes h where the output
+    # is consumed
     for L, pairs, need, out in (("L4", S2, S2, C2), ("L5", S2, S2p, C2),
                                 ("L6", S3p, S3p, C3), ("L7", S3p, S3pp, C3)):
         byts[f"{L}.apply"] = F * pairs * out * 2
@@ -307,16 +307,27 @@ def cpu_baseline(stub_dir, rec, budget_s=15.0, H2=16, W2=20, gpu_out=None):
     return res
 
 
+def launch_work(flops, byts, iface):
+    """The work of algorithmic_work per launch: a layer's projection and
+    recurrence are one launch (k_pscan, timed in the proj slot), whose [v | g]
+    rows pass through LDS and so leave its interface bytes (they are twice
+    the recurrence's state read and write, once written and once read)."""
+    flops, byts, iface = dict(flops), dict(byts), dict(iface)
+    for L in ("L4", "L5", "L6", "L7"):
+        rows = byts[f"{L}.apply"]                  # pairs x 2 OUT floats
+        iface[f"{L}.proj"] += iface.pop(f"{L}.apply") - 2 * rows
+        flops[f"{L}.proj"] += flops.pop(f"{L}.apply")
+        byts[f"{L}.proj"] += byts.pop(f"{L}.apply")
+    return flops, byts, iface
+
+
 # kernel of each timed launch of the whole-ring drain (ssla-rt_amd/csrc/drain_scan.hip)
 PHASE_KERNEL = {"order": "ordering kernels", "head": "k_head + k_pred_*", "emit": "k_emit"}
 for _L, (_i, _o) in zip(("L4", "L5", "L6", "L7"), ((C1, C2), (C2, C2), (C2, C3), (C3, C3))):
-    PHASE_KERNEL[f"{_L}.proj"] = f"k_qvg<{_i}, {_o}>"
-    # the recurrence is one launch (k_scan, in the apply slot); the sum slot
-    # holds L4's wait for the s2 ticket order (L6's for the s3 one comes
-    # before its projection), carry nothing
-    PHASE_KERNEL[f"{_L}.sum"] = "(wait for k_group_order)" if _L == "L4" else "(none)"
-    PHASE_KERNEL[f"{_L}.carry"] = "(none)"
-    PHASE_KERNEL[f"{_L}.apply"] = f"k_scan<{_o}, {_o if _o == C2 else 2 * _o}>"
+    # projection and recurrence are one launch, in the proj slot
+    PHASE_KERNEL[f"{_L}.proj"] = f"k_pscan<{_i}, {_o}>"
+    for _s in ("sum", "carry", "apply"):
+        PHASE_KERNEL[f"{_L}.{_s}"] = "(none)"
     PHASE_KERNEL[f"{_L}.out"] = f"k_outt<{_i}, {_o}>"
 RIDGE = PEAK_FP32_TFLOPS * 1e12 / (PEAK_HBM_GBS * 1e9)     # FLOP/B
 
@@ -609,15 +620,14 @@ def batch_bench(a, d, recs, n, S, steps, warmup, desc, tmp) -> int:
 # launched twice per call belong to the two layers in turn; the ordering
 # kernels are summed into "order"
 TRAFFIC_PHASES = {
-    "k_qvg<24, 48>": ["L4.proj"], "k_qvg<48, 48>": ["L5.proj"], "k_qvg<48, 96>": ["L6.proj"],
-    "k_qvg<96, 96>": ["L7.proj"],
-    "k_scan<48, 48>": ["L4.apply", "L5.apply"], "k_scan<96, 192>": ["L6.apply", "L7.apply"],
+    "k_pscan<24, 48>": ["L4.proj"], "k_pscan<48, 48>": ["L5.proj"], "k_pscan<48, 96>": ["L6.proj"],
+    "k_pscan<96, 96>": ["L7.proj"],
     "k_outt<24, 48, 2, 1>": ["L4.out"], "k_outt<48, 48, 1, 3>": ["L5.out"],
     "k_outt<48, 96, 1, 3>": ["L6.out"], "k_outt<96, 96, 1, 3>": ["L7.out"],
     "k_head": ["head"], "k_head_linear": ["head"], "k_pred_write": ["head"], "k_emit": ["emit"],
 }
 ORDER_KERNELS = ("k_decode", "k_rs_hist", "k_exscan", "k_rs_scatter", "k_runs", "k_keys2",
-                 "k_keyscan", "k_s2_tables", "k_pair_rank", "k_chunks", "k_keys3a", "k_place3",
+                 "k_keyscan", "k_s2_tables", "k_pair_rank", "k_key_groups", "k_keys3a", "k_place3",
                  "k_tdrop3", "k_keys3b", "k_group_order")
 
 
@@ -932,6 +942,7 @@ def main() -> int:
             for k, v in src.items():
                 dst[k] = dst.get(k, 0.0) + v
         total_mac += m_
+    flops, byts, ibyts = launch_work(flops, byts, ibyts)
     roof = _roofline(per_timed, flops, byts, ibyts, roof_phase)
     if a.workload != "80x64":
         roof["traffic"] = None           # the committed PMC summary is of the 80x64 workload
@@ -952,7 +963,7 @@ def main() -> int:
     roof["bytes_note"] = ("achieved / frac: the algorithmic bytes or FLOPs of the launch (for a "
                           "recurrence, each pair's hidden-state read and write); interface_*: "
                           "the bytes it moves at its interface, which include this design's "
-                          "own pair rows and h rows; traffic: the committed PMC measurement")
+                          "own h rows; traffic: the committed PMC measurement")
     whole = 2.0 * total_mac / (ms_step * 1e-3) / 1e12
     iface = sum(ibyts.values())
     comp = sum(compulsory_bytes(r.x, r.y, o["pass2"], H2, W2) for r, o in zip(recs, outs))
@@ -975,7 +986,7 @@ def main() -> int:
         "measured_over_compulsory": round(measured / comp, 3) if measured else None,
         "whole_drain_compulsory_hbm_gbs": round(comp / (ms_step * 1e-3) / 1e9, 1),
         # the bytes every launch moves at its interface, including the design's
-        # own intermediates (pair rows, h rows, chunk maps): not compulsory
+        # own intermediates (h rows): not compulsory
         "whole_drain_launch_interface_gbs": round(iface / (ms_step * 1e-3) / 1e9, 1),
         "phase_ms": {k: round(v, 5) for k, v in per.items()},
         "phase_ms_note": "HIP-event time per phase from an extra loop of the same steps with "
@@ -987,7 +998,7 @@ def main() -> int:
         "roofline_by_phase_note": "per launch against its bound, on its algorithmic bytes or "
                                   "FLOPs; interface_gbs: the rate on the bytes it moves at its "
                                   "interface, which include the design's own intermediates "
-                                  "(pair rows, h rows)",
+                                  "(h rows)",
         "roofline_by_phase": {
             k: {x: r[x] for x in ("bound", "achieved", "unit", "frac", "interface_gbs")}
             for k, r in ((k, _roofline(per, flops, byts, ibyts, k)) for k in per

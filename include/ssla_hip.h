@@ -149,13 +149,12 @@ int ssla_hip_drain_n2(const HybridS2S3Config* cfg,
 
 #define SSLA_DRAIN_PHASES 23
 /* Phase order of SslaHipDrainOpts.phase_ms (one kernel launch each, except
- * 0, 21): 0 ordering (decode, sorts, tdrop decisions, chunk tables); per
- * layer a projection of v, g, the recurrence in three slots, then the
- * contraction (q, q*h, goW, residual, LayerNorm): L4 1-5, L5 6-10, L6
- * 11-15, L7 16-20; 21 head and prediction grid, 22 output slots.  The
- * recurrence of every layer is one launch, in the third of its slots; the
- * first holds L4's wait for its ticket order (built beside L4's
- * projection) and is empty for L5-L7, and the second is empty. */
+ * 0, 21): 0 ordering (decode, sorts, tdrop decisions, pair and group
+ * tables); per layer the projection of v, g with the recurrence over them in
+ * the first of four slots (the other three are empty), then the contraction
+ * (q, q*h, goW, residual, LayerNorm): L4 1-5, L5 6-10, L6 11-15, L7 16-20;
+ * 21 head and prediction grid, 22 output slots.  L6's first slot also holds
+ * the wait for the s3 ordering. */
 
 #define SSLA_BATCH_PHASES 32
 /* Slots of the in-kernel batch profile (batch-mode and live drains), summed
@@ -223,7 +222,7 @@ int ssla_hip_drain_batch_noalloc(const HybridS2S3Config* cfg,
                                  void* stream, int sync);
 
 /* The whole-ring drain keeps one workspace per process (device memory
- * sized for the largest call so far; about 9 KB per record).  A call with
+ * sized for the largest call so far; about 5 KB per record).  A call with
  * more records than it holds regrows it, which waits for the previous
  * drain call to finish and frees and allocates device memory.  Call this
  * once up front -- in particular before ssla_hip_persistent_start, while no

@@ -73,8 +73,13 @@ inline const char* head_missing(const HybridS2S3Config* cfg) {
     return nullptr;
 }
 
+// 1 / (1 + exp(-x)): the reciprocal by v_rcp_f32 and one Newton step, whose
+// infinite and NaN cases v_div_fixup_f32 sets right (7 instructions; the full
+// division that __fdividef compiles to takes 14).
 __device__ __forceinline__ float sigmoid_fast(float x) {
-    return __fdividef(1.0f, 1.0f + __expf(-x));
+    const float d = 1.0f + __expf(-x);
+    const float r = __builtin_amdgcn_rcpf(d);
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, r, 1.0f), r, r), d, 1.0f);
 }
 
 // Bit 31 of a prediction cell's version marks a write in progress.

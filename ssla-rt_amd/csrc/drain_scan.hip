@@ -13,16 +13,15 @@
 //   y_e = LN( sum_delta goW[delta] qh + residual(x_e) )
 //
 // Only the h_c recurrence is ordered, and only among events touching the
-// same cell.  Per layer the drain therefore runs three phases over all
-// records of all rings:
-//   P  (k_qvg)   v, g for every (record, delta) pair as MFMA tiles,
-//                written in per-cell ring order (pair rows sorted by
-//                target cell)
-//   S  (k_scan)  chunked per-cell scan: turns (v, g) rows into h rows in
-//                place, in ring order, where the layer's output is used
-//   O  (k_out)   per output record: q = qvgIn[delta] x by MFMA, times the
-//                <= 9 h rows, contracted with goW by MFMA, residual, fp64
-//                LayerNorm
+// same cell.  Per layer the drain therefore runs two kernels over all records
+// of all rings:
+//   P, S (k_pscan)  v, g for every (record, delta) pair as MFMA tiles, and the
+//                   recurrence over them: groups of pairs in per-cell ring
+//                   order, chained by a look-back scan; writes the h rows
+//                   where the layer's output is used
+//   O    (k_outt)   per output record: q = qvgIn[delta] x by MFMA, times the
+//                   <= 9 h rows, contracted with goW by MFMA, residual, fp64
+//                   LayerNorm
 // The temporal-dropout decisions (ssla_ref.py:190-195) depend only on the
 // per-cell arrival rank of a record, so they come from a stable sort of
 // records by cell: pass = ((counter + rank) mod 256) % window == 0.
@@ -310,28 +309,142 @@ __global__ void __launch_bounds__(kScanThreads) k_exscan(int n, int* __restrict_
     }
 }
 
-constexpr int kCH = 32;     // pairs per scan chunk
-constexpr int kSG = 8;      // chunks per group (workgroup) of the one-pass scan, s2 layers
-constexpr int kSG3 = 4;     // ... s3 layers (two waves per chunk)
+// Groups of the projection + scan kernel (k_pscan): a cell with more than
+// kGW pairs is cut into groups of kGP of its own; cells with fewer share one,
+// all those whose run starts in the same window of kGW pair positions (runs
+// of the pair order are contiguous, and a cell that starts in a window behind
+// a larger one starts in a later window, so a shared group is one range of at
+// most 2 kGW - 1 pairs).
+constexpr int kGP = 176;        // pairs per group (k_pscan: 4 row blocks of 44 per channel)
+constexpr int kGW = kGP / 2;
 
-// Chunk tables: one wave per key writes its chunks (ckey, cbeg, cend) and
-// counts the key's groups of the one-pass scan (ghist, gw: k_group_order).
-__global__ void __launch_bounds__(256)
-k_chunks(uint32_t nk, const int* __restrict__ start, const int* __restrict__ end,
-         const int* __restrict__ coff, int* __restrict__ ckey, int* __restrict__ cbeg,
-         int* __restrict__ cend, int* __restrict__ ghist, int* __restrict__ gw) {
-    const uint32_t k = blockIdx.x * 4u + (threadIdx.x >> 6);
+// group list entry: {first pair, pairs | flags, published-word slot, rank in the cell}
+constexpr int kGStart = 1 << 16;    // the group's first pair is its cell's first
+constexpr int kGEnd = 1 << 17;      // the group's last pair is its cell's last
+constexpr int kGMulti = 1 << 18;    // the group holds several cells
+
+// first index in [lo, hi) of the ascending array a whose value is >= v, else hi
+__device__ __forceinline__ int lower_bound_i(const int* a, int lo, int hi, int v) {
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (a[mid] < v) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// The groups that key k leads (pst: nk + 1 pair starts): its count, and the
+// end of their pair range.
+__device__ __forceinline__ int key_groups(int k, int nk, const int* pst, int* pend) {
+    const int s = pst[k], e = pst[k + 1], n = e - s;
+    *pend = e;
+    if (n == 0) return 0;
+    if (n > kGW) return (n + kGP - 1) / kGP;
+    const int w0 = s - s % kGW;
+    if (pst[lower_bound_i(pst, 0, k, w0)] != s) return 0;     // an earlier cell of the window leads
+    const int kb = lower_bound_i(pst, k + 1, nk, min(w0 + kGW, pst[nk]));
+    // key kb - 1 is the last with pairs that starts in the window
+    *pend = pst[kb] - pst[kb - 1] > kGW ? pst[kb - 1] : pst[kb];
+    return 1;
+}
+
+// Per key, for the keys k_keyscan has no room for in LDS: the groups it leads
+// (gcnt), the end of their range (gend) and its place among the keys with as
+// many (ghist counts them).
+__device__ __forceinline__ void key_group_at(uint32_t k, uint32_t nk, const int* __restrict__ pst,
+                                             int* __restrict__ gcnt, int* __restrict__ gend,
+                                             int* __restrict__ ghist, int* __restrict__ gw) {
     if (k >= nk) return;
-    const int s = start[k], e = end[k], c0 = coff[k];
-    for (int q = threadIdx.x & 63; s + q * kCH < e; q += 64) {
-        ckey[c0 + q] = (int)k;
-        cbeg[c0 + q] = s + q * kCH;
-        cend[c0 + q] = min(e, s + (q + 1) * kCH);
+    int pend;
+    const int gc = key_groups((int)k, (int)nk, pst, &pend);
+    gcnt[k] = gc;
+    gend[k] = pend;
+    if (gc > 0) gw[k] = atomicAdd(&ghist[gc], 1);
+}
+
+__global__ void __launch_bounds__(256)
+k_key_groups(uint32_t nk, const int* __restrict__ pst, int* __restrict__ gcnt,
+             int* __restrict__ gend, int* __restrict__ ghist, int* __restrict__ gw) {
+    key_group_at(blockIdx.x * 256u + threadIdx.x, nk, pst, gcnt, gend, ghist, gw);
+}
+
+// The ticket order of the groups (one workgroup): tickets take every cell's
+// group 0, then every cell's group 1, ..., cells with more groups first, so
+// a group's predecessors in its cell hold smaller tickets.  hist[v] counts the
+// keys that lead v groups (nv entries) and place(k) is key k's place among
+// them.  start[v] = keys with more than v groups (the groups of rank v),
+// base[r] = tickets before rank r; key k, at place start[gc] + place of every
+// rank below gc, gets glist[base[r] + start[gc] + place] for its rank r.
+// lead(k) -> (group count, range end, place, first pair, first slot).
+struct LeadKey {
+    int gc, pend, place, p0, slot, multi;
+};
+template <class Lead>
+__device__ __forceinline__ void group_order(int nk, int nv, const int* hist, int* start, int* base,
+                                            int* lds, Lead lead, int4* __restrict__ glist,
+                                            int* __restrict__ n_groups) {
+    int carry = 0;
+    for (int r0 = 0; r0 < nv; r0 += kScanRound) {        // start: scan of hist from the top
+        const int i0 = r0 + (int)threadIdx.x * kScanPer;
+        int v[kScanPer], sum = 0;
+        #pragma unroll
+        for (int q = 0; q < kScanPer; ++q) {
+            v[q] = i0 + q < nv ? hist[nv - 1 - (i0 + q)] : 0;
+            sum += v[q];
+        }
+        int total;
+        int run = carry + block_exscan(sum, lds, &total);
+        carry += total;
+        #pragma unroll
+        for (int q = 0; q < kScanPer; ++q) {
+            if (i0 + q < nv) start[nv - 1 - (i0 + q)] = run;
+            run += v[q];
+        }
     }
-    if ((threadIdx.x & 63) == 0) {
-        const int gc = ((e - s + kCH - 1) / kCH + kSG3 - 1) / kSG3;
-        if (gc > 0) gw[k] = atomicAdd(&ghist[gc], 1);
+    __syncthreads();
+    carry = 0;
+    for (int r0 = 0; r0 < nv; r0 += kScanRound) {        // base: prefix of start
+        const int i0 = r0 + (int)threadIdx.x * kScanPer;
+        int v[kScanPer], sum = 0;
+        #pragma unroll
+        for (int q = 0; q < kScanPer; ++q) {
+            v[q] = i0 + q < nv ? start[i0 + q] : 0;
+            sum += v[q];
+        }
+        int total;
+        int run = carry + block_exscan(sum, lds, &total);
+        carry += total;
+        #pragma unroll
+        for (int q = 0; q < kScanPer; ++q) {
+            if (i0 + q < nv) base[i0 + q] = run;
+            run += v[q];
+        }
     }
+    if (threadIdx.x == 0) *n_groups = carry;
+    __syncthreads();
+    for (int k = threadIdx.x; k < nk; k += kScanThreads) {
+        const LeadKey L = lead(k);
+        const int p = L.gc > 0 ? start[L.gc] + L.place : 0;
+        for (int r = 0; r < L.gc; ++r) {
+            const int p0 = L.p0 + r * kGP;
+            glist[base[r] + p] = make_int4(p0, min(kGP, L.pend - p0) | (r == 0 ? kGStart : 0) |
+                                                   (r == L.gc - 1 ? kGEnd : 0) | L.multi,
+                                           L.slot + r, r);
+        }
+    }
+}
+
+// The same from the tables in global memory (any number of keys and groups).
+__global__ void __launch_bounds__(kScanThreads)
+k_group_order(int nk, int nv, const int* __restrict__ pst, const int* __restrict__ goff,
+              const int* __restrict__ gcnt, const int* __restrict__ gend, const int* ghist,
+              const int* __restrict__ gw, int* gstart, int* gbase, int4* __restrict__ glist,
+              int* __restrict__ n_groups) {
+    __shared__ int lds[2 * (kScanThreads / 64)];
+    group_order(nk, nv, ghist, gstart, gbase, lds, [&](int k) {
+        return LeadKey{gcnt[k], gend[k], gw[k], pst[k], goff[k],
+                       gend[k] > pst[k + 1] ? kGMulti : 0};
+    }, glist, n_groups);
 }
 
 // [start, end) of every key present in a sorted key array.
@@ -457,19 +570,35 @@ __device__ __forceinline__ void key2_at(uint32_t t, const KeyHist& kh, int& pc, 
 }
 
 // Per-key tables from per-key counts (k < nk), in one launch:
-//   cnt  -> start (exclusive scan), end = start + cnt (end may be cnt itself);
-//           with coff: coff[k] = the key's first chunk of kCH, *n_chunks;
+//   cnt  -> start (exclusive scan, nk + 1 values), end = start + cnt (optional;
+//           end may be cnt itself);
+//           with goff: goff[k] = the key's first published-word slot (one per
+//           kGP pairs);
 //   cnt2 (optional) -> off2 (exclusive scan), *total2.
 // KH: the counts come from key2_at (a one-pass sort's histogram, kh; nk <=
 // kScanThreads) instead of cnt / cnt2, and cnt2 then receives the pass-2
 // counts.
-template <bool KH>
+// GT: the group list too (nk <= kScanThreads keys and gt.nv <= kGroupLds group
+// counts, all tables in LDS), which a call with few keys would otherwise wait
+// for two more launches for.
+constexpr int kGroupLds = 6144;
+struct GroupTab {
+    int nv;
+    int4* glist;
+    int* n_groups;
+};
+
+template <bool KH, bool GT>
 __global__ void __launch_bounds__(kScanThreads)
-k_keyscan(int nk, const int* cnt, int* __restrict__ start, int* end, int* __restrict__ coff,
-          int* __restrict__ n_chunks, const int* __restrict__ cnt2, int* __restrict__ off2,
-          int* __restrict__ total2, KeyHist kh) {
+k_keyscan(int nk, const int* cnt, int* __restrict__ start, int* end, int* __restrict__ goff,
+          const int* __restrict__ cnt2, int* __restrict__ off2,
+          int* __restrict__ total2, KeyHist kh, GroupTab gt) {
     __shared__ int lds[2 * (kScanThreads / 64)];
     __shared__ int kv[KH ? kScanThreads : 1], ku[KH ? kScanThreads : 1];
+    __shared__ int spst[GT ? kScanThreads + 1 : 1], sgo[GT ? kScanThreads : 1];
+    __shared__ int shist[GT ? kGroupLds : 1], sstart[GT ? kGroupLds : 1];
+    if constexpr (GT)
+        for (int i = threadIdx.x; i < gt.nv; i += kScanThreads) shist[i] = 0;
     int carry = 0, ccarry = 0, carry2 = 0;
     for (int r0 = 0; r0 < nk; r0 += kScanRound) {
         const int i0 = r0 + (int)threadIdx.x * kScanPer;
@@ -500,7 +629,7 @@ k_keyscan(int nk, const int* cnt, int* __restrict__ start, int* end, int* __rest
         #pragma unroll
         for (int q = 0; q < kScanPer; ++q) {
             s += v[q];
-            c[q] = (v[q] + kCH - 1) / kCH;
+            c[q] = (v[q] + kGP - 1) / kGP;
             sc += c[q];
             if (cnt2) su += u[q];
         }
@@ -508,7 +637,7 @@ k_keyscan(int nk, const int* cnt, int* __restrict__ start, int* end, int* __rest
         int run = carry + block_exscan(s, lds, &total);
         carry += total;
         int crun = 0, urun = 0;
-        if (coff) {
+        if (goff) {
             crun = ccarry + block_exscan(sc, lds, &total);
             ccarry += total;
         }
@@ -528,15 +657,34 @@ k_keyscan(int nk, const int* cnt, int* __restrict__ start, int* end, int* __rest
             const int y = u[q];
             u[q] = urun;
             urun += y;
+            if constexpr (GT) {
+                if (i0 + q < nk) {
+                    spst[i0 + q] = st[q];
+                    sgo[i0 + q] = c[q];
+                }
+            }
         }
         store8(start, i0, nk, st);
-        store8(end, i0, nk, en);
-        if (coff) store8(coff, i0, nk, c);
+        if (end) store8(end, i0, nk, en);
+        if (goff) store8(goff, i0, nk, c);
         if (cnt2) store8(off2, i0, nk, u);
     }
     if (threadIdx.x == 0) {
-        if (coff) *n_chunks = ccarry;
+        start[nk] = carry;
         if (cnt2) *total2 = carry2;
+    }
+    if constexpr (GT) {
+        if (threadIdx.x == 0) spst[nk] = carry;
+        __syncthreads();
+        const int k = (int)threadIdx.x;
+        int gc = 0, pend = 0, place = 0;
+        if (k < nk) gc = key_groups(k, nk, spst, &pend);
+        if (gc > 0) place = atomicAdd(&shist[gc], 1);
+        __syncthreads();
+        // (the base table takes hist's place: hist is read before it is written)
+        group_order(nk, gt.nv, shist, sstart, shist, lds, [&](int q) {
+            return LeadKey{gc, pend, place, spst[q], sgo[q], pend > spst[q + 1] ? kGMulti : 0};
+        }, gt.glist, gt.n_groups);
     }
 }
 
@@ -684,14 +832,14 @@ __global__ void k_keys3b(uint32_t nk3, Geometry G, const int* __restrict__ t3,
 // One thread per sorted record i (record g = vals[i], key k = keys[i]): the
 // ranks of g in the 5 x 5 runs around its centre cell (its own run gives
 // i - st[k]), folded row by row into three horizontal 3-sums; a delta's rank
-// is the sum of three of them.  pos[g * 9 + d] = the pair's place in the pair
-// order (-1 when the target is off the grid or the record has no key), and
-// pair_need[place] = whether g needs the layer's output (pass[g], or `take`
-// when pass is null: the tdrop decision the same thread just made), so the
-// scan's apply pass reads one byte per pair in its own order instead of a
-// record id and then that record's flag.  The lanes of a wave that share a
-// centre cell (records are sorted by cell) rank together: every load then
-// serves the whole segment, which keeps the L2 request count low.
+// is the sum of three of them.  The pair's entry at its place in the pair
+// order is {9 g + d, t's key}, with kPairNeed set in the id when g needs the
+// layer's output (pass[g], or `take` when pass is null: the tdrop decision the
+// same thread just made), so k_pscan reads all it needs of a pair in its own
+// order.  The lanes of a wave that share a centre cell (records are sorted by
+// cell) rank together: every load then serves the whole segment, which keeps
+// the L2 request count low.
+constexpr uint32_t kPairNeed = 0x80000000u;      // (9 records fit 31 bits)
 constexpr int kSegMax = 4;   // cell segments of a wave ranked together; more: per lane
 constexpr int kChunkWide = 512;   // widest window counted in 64-value chunks
 
@@ -812,8 +960,7 @@ __device__ __forceinline__ void
 pair_rank_at(int i, int n, const uint32_t* __restrict__ keys,
              const uint32_t* __restrict__ vals, uint32_t nk, int C, int W, int H,
              const int* __restrict__ st, const int* __restrict__ en, const int* __restrict__ pst,
-             int* __restrict__ pos, unsigned char* __restrict__ pair_need,
-             const unsigned char* __restrict__ pass, bool take) {
+             uint2* __restrict__ pent, const unsigned char* __restrict__ pass, bool take) {
     const int lane = threadIdx.x & 63;
     const bool valid = i < n;
     const uint32_t k = valid ? keys[i] : nk;
@@ -868,15 +1015,9 @@ pair_rank_at(int i, int n, const uint32_t* __restrict__ keys,
         #pragma unroll
         for (int c = 0; c < 25; ++c) r25[c] = lo[c] - r25[c];
     }
-    if (!valid) return;
-    int* pg = pos + (size_t)g * kPatch;
-    if (k >= nk) {
-        #pragma unroll
-        for (int d = 0; d < kPatch; ++d) pg[d] = -1;
-        return;
-    }
+    if (!keyed) return;
     const int b = (int)k / C, cell = (int)k % C, y = cell / W, x = cell % W;
-    const unsigned char need = pass ? pass[g] : (unsigned char)take;
+    const uint32_t need = (pass ? pass[g] != 0 : take) ? kPairNeed : 0u;
     r25[12] = i - st[k];
     int hs[5][3];                  // hs[row][dx + 1]: runs (row, dx - 1 .. dx + 1)
     #pragma unroll
@@ -888,14 +1029,10 @@ pair_rank_at(int i, int n, const uint32_t* __restrict__ keys,
     for (int d = 0; d < kPatch; ++d) {
         const int dy = 1 - d / 3, dx = 1 - d % 3;      // target offset from the centre
         const int ty = y + dy, tx = x + dx;
-        if (ty < 0 || ty >= H || tx < 0 || tx >= W) {
-            pg[d] = -1;
-            continue;
-        }
+        if (ty < 0 || ty >= H || tx < 0 || tx >= W) continue;
         const int rank = hs[dy + 1][dx + 1] + hs[dy + 2][dx + 1] + hs[dy + 3][dx + 1];
-        const int p = pst[b * C + ty * W + tx] + rank;
-        pg[d] = p;
-        pair_need[p] = need;
+        const int t = b * C + ty * W + tx;
+        pent[pst[t] + rank] = make_uint2((g * kPatch + d) | need, (uint32_t)t);
     }
 }
 
@@ -903,73 +1040,87 @@ __global__ void __launch_bounds__(256)
 k_pair_rank(int n_max, const int* __restrict__ n_dev, const uint32_t* __restrict__ keys,
             const uint32_t* __restrict__ vals, uint32_t nk, int C, int W, int H,
             const int* __restrict__ st, const int* __restrict__ en, const int* __restrict__ pst,
-            int* __restrict__ pos, unsigned char* __restrict__ pair_need,
-            const unsigned char* __restrict__ pass) {
+            uint2* __restrict__ pent, const unsigned char* __restrict__ pass) {
     pair_rank_at(blockIdx.x * blockDim.x + threadIdx.x, n_dev ? *n_dev : n_max, keys, vals, nk,
-                 C, W, H, st, en, pst, pos, pair_need, pass, false);
+                 C, W, H, st, en, pst, pent, pass, false);
 }
 
 // The s2 level's tables that need only the sorted order and the key scan, in
 // one launch: per sorted record (blocks [0, nbr)) its tdrop_s2 decision and
-// list slot (k_tdrop2) and its pair ranks (k_pair_rank); per key (blocks
-// nbr.., one wave each) its chunk table (k_chunks).
+// list slot (tdrop2_at) and its pair ranks; per key (blocks nbr.., when the key
+// scan did not build the group list) the groups it leads.
 __global__ void __launch_bounds__(256)
 k_s2_tables(int n, int nbr, const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,
             uint32_t nk, int C, int W, int H, const int* __restrict__ st,
-            const int* __restrict__ en, const int* __restrict__ pst, const int* __restrict__ pen,
-            const int* __restrict__ coff, const unsigned char* __restrict__ old,
+            const int* __restrict__ en, const int* __restrict__ pst,
+            const unsigned char* __restrict__ old,
             const int* __restrict__ off, int window, unsigned char* __restrict__ pass,
-            int* __restrict__ list, int* __restrict__ pos, unsigned char* __restrict__ pair_need,
-            int* __restrict__ ckey, int* __restrict__ cbeg, int* __restrict__ cend,
-            int* __restrict__ ghist, int* __restrict__ gw) {
+            int* __restrict__ list, uint2* __restrict__ pent, int* __restrict__ gcnt,
+            int* __restrict__ gend, int* __restrict__ ghist, int* __restrict__ gw) {
     if ((int)blockIdx.x >= nbr) {
-        const uint32_t k = (blockIdx.x - (unsigned)nbr) * 4u + (threadIdx.x >> 6);
-        if (k >= nk) return;
-        const int s0 = pst[k], e = pen[k], c0 = coff[k];
-        for (int q = threadIdx.x & 63; s0 + q * kCH < e; q += 64) {
-            ckey[c0 + q] = (int)k;
-            cbeg[c0 + q] = s0 + q * kCH;
-            cend[c0 + q] = min(e, s0 + (q + 1) * kCH);
-        }
-        // the key's groups of the one-pass scan (k_group_order)
-        if ((threadIdx.x & 63) == 0) {
-            const int gc = ((e - s0 + kCH - 1) / kCH + kSG - 1) / kSG;
-            if (gc > 0) gw[k] = atomicAdd(&ghist[gc], 1);
-        }
+        key_group_at((blockIdx.x - (unsigned)nbr) * 256u + threadIdx.x, nk, pst, gcnt, gend, ghist,
+                     gw);
         return;
     }
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const bool take = tdrop2_at(i, n, keys, vals, nk, st, old, off, window, pass, list);
-    pair_rank_at(i, n, keys, vals, nk, C, W, H, st, en, pst, pos, pair_need, nullptr, take);
+    pair_rank_at(i, n, keys, vals, nk, C, W, H, st, en, pst, pent, nullptr, take);
 }
 
 // ---------------------------------------------------------------------------
-// P: v, g rows as 16 x 16 MFMA tiles (v_mfma_f32_16x16x4_f32, operand layout
-// in mfma_pack.h).  A record tile = 64 records (rows, staged in LDS) x all 9
-// deltas x the v and g column tiles of qvgIn; each wave owns (delta, column
-// tile) items, loads an item's weights (fragment order, one float4 per four
-// k-steps) while the previous item's four row tiles run, and writes each
-// [v | g] row (2 * OUT floats) to the pair's sorted position.  q is not
-// stored: the contraction recomputes it from the record's input.  With the
-// weights as the A operand a lane's four results are four consecutive
-// channels of one record, stored as one 16-byte piece of its row (staging
-// whole rows across waves measured slower: the barriers cost more than the
-// partial-line writes).
+// P + S: projection and recurrence in one kernel (k_pscan).  Per layer, every
+// (record, delta) pair needs v, g = x_record Wvg[delta] and then
+// h = sigmoid(g) h + v along its cell's pairs in ring order.  A workgroup (one
+// per CU, 16 waves, persistent) takes groups of up to kGP pairs of the pair
+// order (see key_groups) and 48 of the layer's channels at a time; its waves
+// have roles and hand groups on through LDS counters (PsSlot), with up to four
+// groups in flight:
+//   deal (1 wave)   draws tickets two ahead, loads a group's pairs and deals
+//     them into 16-pair MFMA tiles of one delta each (a tile's missing pairs
+//     repeat a record and write a spare row);
+//   tiles (8 waves, two per SIMD)   per tile the records' input rows are the B
+//     operand (one float4 per lane and four k-steps, straight from the feature
+//     rows, the next tile's while a tile runs) and the delta's weights the A
+//     operand (fragment order, ProjPackT, streamed DW - 1 parts ahead), so a
+//     lane's four results are four channels of one pair: v and sigmoid(g) go to
+//     the pair's row in LDS.  The [v | g] rows never reach memory;
+//   rows (two teams of 3 waves, every other group each)   thread (sub, channel)
+//     takes kPSRows consecutive rows into registers, which frees the LDS buffer
+//     for the group after the next, and composes their map h -> A h + B (a cell's
+//     first pair has its cell's stored state folded in: A = 0); with its start
+//     state it replays them, writes h at row 9 g + d where the pair's record
+//     needs the layer's output (a record's nine rows are contiguous for its
+//     contraction), and stores the state of a cell's last pair;
+//   chain (1 wave)   composes the group's map and finds its start state: none
+//     needed for a group that begins with a cell's first pair, else by looking
+//     back over the cell's earlier groups -- the nearest one whose end state is
+//     published, then the maps of the groups after it, applied forward.  A group
+//     publishes its map before it waits and its end state once it has its start,
+//     so every state is the same fixed chain of fmaf's whichever word a reader
+//     happens to find: the results do not depend on timing.
+// Tickets: group_order lists a group's predecessors in its cell before it.  A
+// workgroup holds several tickets, works on them in ascending order and waits
+// only for smaller ones, so the smallest unfinished ticket never waits.
+// Published words hold a float and the launch's tag (value | tag << 32) and are
+// stored and loaded with relaxed device-scope atomics: a reader that sees the
+// tag sees the value, with no fence (a release fence would write back the L2).
+// Every wait on another workgroup is bounded on the wall clock; a wave that runs
+// out raises *err (host memory) and goes on with a zero state.
 //
-// PT (the layers over all records): a workgroup loops over record tiles
-// (tile += gridDim.x) and loads the next tile's rows and pair positions into
-// registers while the current tile runs, so the load latency of a tile is
-// not paid at the start of a workgroup.  The tiles are 80 records and the
-// grid is sized per layer from the CU count (scan_drain) so that each
-// workgroup runs about two of them; the launch bounds ask for 5 waves per
-// SIMD (L5: 4 waves to 5).  The pass-2 layers keep one 64-record tile per
-// workgroup: the prefetch registers cost L7 (IN = 96) a wave per SIMD.
-// Their tiles are few (the pass-2 records: ~800 tiles at 200k), so NP
-// workgroups share a tile, each running 1/NP of its items (L6: 2, L7: 4):
-// with 3-4 tiles per CU, a third of the CUs had one more tile than the rest.
+// Bounds and measurements (200k records at 80 x 64, L4 / L5 / L6 / L7): the fp32
+// matrix cores need 67 / 135 / 62 / 127 us for the tiles (11 pairs of a tile's 16
+// are real: 9 deltas share a group's 176 pairs), and were busy 35-52% of 0.20 /
+// 0.28 / 0.155 / 0.235 ms.  The two launches this replaced (projection to pair
+// rows in memory, one-pass scan over them) took 0.41 / 0.38 / 0.22 / 0.26 ms and
+// moved 4 GB more per call; the drain went 1.80 -> 1.40 ms.  Loads are not the
+// bound (rows or weights from the L1 changed the times by 2-8%).  Measured on the
+// way: workgroups of 6 waves do not pair on a CU (2.05 ms per call); 8 waves that
+// run all phases in turn, two workgroups per CU, 1.70; the same with look-back
+// and replay of a group behind the tiles of the next, 1.52; one row team of 3
+// waves and 11 tile waves, 1.51; two interleaved accumulator chains per tile
+// wave, 1.43 (a single dependent chain forwards its accumulator).
 // ---------------------------------------------------------------------------
-constexpr int kTM = 64;     // records per projection / contraction workgroup
-constexpr int kTMP = 80;    // records per tile of the persistent projection
+constexpr int kTM = 64;     // records per head workgroup
 
 // Row stride of the LDS tiles read as MFMA A operands, a[(16 m + li) ST + lk
 // + 4 s] with li = lane % 16, lk = lane / 16: a stride of 2 (mod 4) puts the
@@ -982,207 +1133,6 @@ __device__ __forceinline__ void lds_put4(float* p, float4 v) {
     reinterpret_cast<float2*>(p)[1] = make_float2(v.z, v.w);
 }
 
-// The items of one staged record tile of TM records (TM / 16 row tiles; rows
-// past the tile's records are zero in LDS and their pair positions -1), part
-// `part` of NP: items [NI part / NP, NI (part + 1) / NP), wave wv taking every
-// fourth from the part's item wv.  The item loop is unrolled with a fixed trip
-// count and its loads and stores carry no branch: the next item's weights are
-// in flight while the current item runs, and the wait before an item covers
-// only its own loads.  A result row with no pair (position -1) is written to
-// `trash` (one 16-byte slot per lane, never read) instead of being skipped.
-template <int IN, int OUT, int TM, int NP>
-__device__ __forceinline__ void qvg_items(const float* __restrict__ xs, const int (*prow)[TM],
-                                          const float* __restrict__ pp, float* __restrict__ QVG,
-                                          float* __restrict__ trash, int part, int tid) {
-    using P = ProjPack<IN, OUT>;
-    constexpr int XST = lds_stride(IN), NCW = 2 * OUT, MT = TM / kMT, KS = P::KS;
-    constexpr int tlo = P::TQ, nti = P::T - tlo, NI = kPatch * nti;
-    static_assert(NI % NP == 0 && TM % kMT == 0, "item parts, row tiles");
-    constexpr int NPI = NI / NP, KF = NPI / 4, KR = NPI % 4;
-    const int lane = tid & 63, wv = tid >> 6, li = lane & 15, lk = lane >> 4;
-    const int ib = NPI * part + wv;            // this wave's items: ib + 4 k
-    // the weight fragment of an item: KS values per lane, as float4 groups (a
-    // final group of two steps as a float2, so no dead register is in flight)
-    auto load = [&](int k, float (&b)[KS]) {
-        const int it = ib + 4 * k, d = it / nti, t = tlo + (it - d * nti);
-        const SSLA_GLOBAL f32x4* src =
-            (const SSLA_GLOBAL f32x4*)pp + (size_t)(d * P::T + t) * P::KS4 * 64 + lane;
-        #pragma unroll
-        for (int g = 0; g < P::KS4; ++g) {
-            if (KS - 4 * g >= 4) {
-                const f32x4 v = src[g * 64];
-                #pragma unroll
-                for (int j = 0; j < 4; ++j) b[4 * g + j] = v[j];
-            } else {
-                const f32x2 v = *(const SSLA_GLOBAL f32x2*)(src + g * 64);
-                b[4 * g] = v[0];
-                b[4 * g + 1] = v[1];
-            }
-        }
-    };
-    // The weight fragment is the A operand and the records the B operand, so
-    // the 16 x 16 result is (channel, record): lane (li, lk) holds channels
-    // 4 lk .. 4 lk + 3 of record li -- one float4 of that record's row.
-    auto run = [&](int k, const float (&b)[KS]) {
-        const int it = ib + 4 * k, d = it / nti, t = tlo + (it - d * nti);
-        const int c0 = t * kMT - OUT + 4 * lk;
-        #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            const float* a = &xs[(m * kMT + li) * XST + lk];
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            #pragma unroll
-            for (int s = 0; s < KS; ++s)
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(b[s], a[4 * s], acc, 0, 0, 0);
-            const int pr = prow[d][m * kMT + li];
-            float* dst = pr >= 0 ? QVG + (size_t)pr * NCW + c0 : trash + 4 * lane;
-            *(SSLA_GLOBAL f32x4*)dst = acc;
-        }
-    };
-    float bb[2][KS];
-    load(0, bb[0]);
-    #pragma unroll
-    for (int k = 0; k < KF; ++k) {
-        if (k + 1 < KF) load(k + 1, bb[(k + 1) & 1]);
-        else if (wv < KR) load(KF, bb[KF & 1]);
-        __builtin_amdgcn_sched_barrier(0);
-        run(k, bb[k & 1]);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    if (wv < KR) run(KF, bb[KF & 1]);
-}
-
-template <int IN, int OUT, bool PT, int TM = kTM, int NP = 1>
-__global__ void __launch_bounds__(256, PT ? 5 : 1)
-k_qvg(int n_max, const int* __restrict__ n_dev, const int* __restrict__ list,
-      const float* __restrict__ X, const int* __restrict__ pos, const float* __restrict__ pp,
-      float* __restrict__ QVG, float* __restrict__ trash) {
-    constexpr int XST = lds_stride(IN), I4 = IN / 4;
-    __shared__ __align__(16) float xs[TM * XST];
-    __shared__ int prow[kPatch][TM];
-    const int n = n_dev ? *n_dev : n_max;
-    const int ntiles = (n + TM - 1) / TM;
-    int tile = PT ? (int)blockIdx.x : (int)blockIdx.x / NP;
-    if (tile >= ntiles) return;
-    const int tid = threadIdx.x;
-    if constexpr (!PT) {
-        const int base = tile * TM, cnt = min(TM, n - base);
-        for (int t = tid; t < TM * I4; t += 256) {
-            const int r = t / I4, q = t - r * I4;
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (r < cnt) {
-                const int g = list ? list[base + r] : base + r;
-                v = reinterpret_cast<const float4*>(X)[(size_t)g * I4 + q];
-            }
-            lds_put4(&xs[r * XST + 4 * q], v);
-        }
-        for (int t = tid; t < TM * kPatch; t += 256) {
-            const int r = t / kPatch, d = t - r * kPatch;
-            int pr = -1;
-            if (r < cnt) {
-                const int g = list ? list[base + r] : base + r;
-                pr = pos[(size_t)g * kPatch + d];
-            }
-            prow[d][r] = pr;
-        }
-        __syncthreads();
-        qvg_items<IN, OUT, TM, NP>(xs, prow, pp, QVG, trash, (int)blockIdx.x % NP, tid);
-    } else {
-        // this thread's share of a tile: XL float4 of input rows, PL positions
-        constexpr int XL = (TM * I4 + 255) / 256, PL = (TM * kPatch + 255) / 256;
-        float4 xv[XL];
-        int pv[PL];
-        auto fetch = [&](int tl) {
-            const int base = tl * TM, cnt = min(TM, n - base);
-            #pragma unroll
-            for (int j = 0; j < XL; ++j) {
-                const int t = tid + 256 * j, r = t / I4, q = t - r * I4;
-                xv[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (t < TM * I4 && r < cnt) {
-                    const int g = list ? list[base + r] : base + r;
-                    xv[j] = reinterpret_cast<const float4*>(X)[(size_t)g * I4 + q];
-                }
-            }
-            #pragma unroll
-            for (int j = 0; j < PL; ++j) {
-                const int t = tid + 256 * j, r = t / kPatch, d = t - r * kPatch;
-                pv[j] = -1;
-                if (t < TM * kPatch && r < cnt) {
-                    const int g = list ? list[base + r] : base + r;
-                    pv[j] = pos[(size_t)g * kPatch + d];
-                }
-            }
-        };
-        fetch(tile);
-        while (true) {
-            #pragma unroll
-            for (int j = 0; j < XL; ++j) {
-                const int t = tid + 256 * j, r = t / I4, q = t - r * I4;
-                if (t < TM * I4) lds_put4(&xs[r * XST + 4 * q], xv[j]);
-            }
-            #pragma unroll
-            for (int j = 0; j < PL; ++j) {
-                const int t = tid + 256 * j, r = t / kPatch, d = t - r * kPatch;
-                if (t < TM * kPatch) prow[d][r] = pv[j];
-            }
-            __syncthreads();
-            const int next = tile + (int)gridDim.x;
-            if (next < ntiles) fetch(next);
-            // the thread index passes through an empty asm each tile, so the
-            // compiler does not hoist the items' addresses out of the tile
-            // loop (kept live across it, they spilled)
-            int tid_t = tid;
-            asm volatile("" : "+v"(tid_t));
-            qvg_items<IN, OUT, TM, 1>(xs, prow, pp, QVG, trash, 0, tid_t);
-            if (next >= ntiles) break;
-            __syncthreads();          // every wave is done with the tile
-            tile = next;
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// S: the per-cell recurrence h = sigmoid(g) h + v over a cell's pairs in ring
-// order, in one pass (k_scan): each pair's v, g row is read once.  A cell's
-// run is cut into chunks of kCH = 32 pairs and its chunks into groups (kSG = 8
-// at s2, kSG3 = 4 at s3: 256 and 128 pairs); one workgroup takes one group,
-// one wave per chunk and 64 channels (two waves for the 96 channels of L6 and
-// L7):
-//   1. each wave loads its chunk's rows into registers (sigmoid(g) in place,
-//      nontemporal loads: the projection has just left up to 0.7 GB of rows
-//      in the caches) and composes the chunk's map h -> A h + B into LDS;
-//   2. the first chunk's waves compose the group's map (SA, SB) in chunk
-//      order and find the group's start state: the cell's stored state for
-//      its first group, else by looking back over the cell's earlier groups
-//      -- the nearest one whose end state is published, then the maps of the
-//      groups after it, applied forward.  A group publishes its map before it
-//      waits and its end state SA h0 + SB once it has h0, so every state is
-//      the same fixed chain of fmaf's whichever word a reader happens to
-//      find: the results do not depend on timing.  The cell's last group
-//      stores the final state;
-//   3. every wave replays its chunk from registers from its start state and
-//      writes h where the pair's record needs the layer's output (L4, L5: a
-//      compact (pairs, 48) array behind the rows, which their contractions
-//      gather 10% faster, stored nontemporal; L6, L7: over v in place).
-// Workgroups draw tickets, and ticket t is glist[t] (k_group_order): every
-// cell's group 0, then every cell's group 1, ...  A group's predecessors in
-// its cell drew earlier tickets (so they have started, and none of them
-// waits for a later group), and about one rank of groups earlier, so the
-// predecessor has usually published its end state by the time a group
-// looks.  Measured at 200k records against the three passes it replaced
-// (summary, per-cell carry, apply): L4 0.32 -> 0.26 ms, L5 0.28 -> 0.21,
-// L6 0.14 -> 0.14, L7 0.125 -> 0.12; in cell order a cell's groups all ran at
-// once and waited on each other down the chain (L4 0.39 ms).  One chunk per
-// group at s3 (0.14, 0.13 ms), two or eight at s2 (0.27, 0.31 ms) were slower
-// with 64-pair chunks.  Chunks of 32 pairs halve a wave's row registers (123
-// VGPRs, no spill, against 168 and 16 B of scratch): L4 0.27 -> 0.26 ms, L5
-// 0.21 -> 0.20, L6 0.13 -> 0.11, L7 0.107 -> 0.090 (1.86 -> 1.80 ms per call);
-// 16-chunk groups (1024 threads) and 16-pair chunks were slower.
-// Published words hold a float and the launch's tag (value | tag << 32)
-// and are stored and loaded with relaxed device-scope atomics: a reader that
-// sees the tag sees the value, with no fence (a release fence would write
-// back the L2).  Every wait is bounded on the wall clock; a wave that runs
-// out raises *err (host memory) and goes on with a zero state.
-// ---------------------------------------------------------------------------
 constexpr int kLB = 4;       // groups looked at per look-back step
 
 __device__ __forceinline__ void sw_put(unsigned long long* p, float v, unsigned tag) {
@@ -1201,13 +1151,13 @@ __device__ __forceinline__ float sw_val(unsigned long long x) {
 
 // Start state of the group of rank r > 0 of a cell (channel cc of a lane;
 // `on` marks the lanes that carry a channel).  The cell's group of rank x
-// publishes [end | SA | SB] x OUT words at sw + (slot0 + x kSG) 3 OUT; rank
-// 0 publishes its end state without waiting.
-template <int OUT, int SG>
+// publishes [end | SA | SB] x OUT words at sw + (slot0 + x) 3 OUT; rank 0
+// publishes its end state without waiting.
+template <int OUT>
 __device__ float scan_lookback(const unsigned long long* __restrict__ sw, int slot0, int r, int cc,
                                bool on, unsigned tag, unsigned long long deadline,
                                int* __restrict__ err) {
-    auto word = [&](int x) { return sw + ((size_t)slot0 + (size_t)x * SG) * 3 * OUT + cc; };
+    auto word = [&](int x) { return sw + ((size_t)slot0 + (size_t)x) * 3 * OUT + cc; };
     // phase 1: the nearest group whose end state every lane sees
     int top = r - 1, found = -1;
     float h = 0.f;
@@ -1229,7 +1179,8 @@ __device__ float scan_lookback(const unsigned long long* __restrict__ sw, int sl
             continue;
         }
         if ((unsigned long long)wall_clock64() > deadline) {
-            if (cc == 0) __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            if ((threadIdx.x & 63) == 0)
+                __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             return 0.f;
         }
         __builtin_amdgcn_s_sleep(2);
@@ -1250,7 +1201,8 @@ __device__ float scan_lookback(const unsigned long long* __restrict__ sw, int sl
             for (int q = 0; q < kLB; ++q) ok = ok && (x0 + q >= r || (sw_ok(a[q], tag) && sw_ok(b[q], tag)));
             if (__all(!on || ok)) break;
             if ((unsigned long long)wall_clock64() > deadline) {
-                if (cc == 0) __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                if ((threadIdx.x & 63) == 0)
+                    __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                 return 0.f;
             }
             __builtin_amdgcn_s_sleep(2);
@@ -1262,192 +1214,435 @@ __device__ float scan_lookback(const unsigned long long* __restrict__ sw, int sl
     return h;
 }
 
-// The one-pass scan's ticket order (one workgroup): a cell's run of nc
-// chunks forms gc = ceil(nc / kSG) groups; tickets take every cell's group
-// 0, then every cell's group 1, ..., cells with more groups first.
-// ghist[v] counts the cells with gc = v and gw[k] is cell k's place among
-// them (k_s2_tables).  start[v] = cells with more than v groups (the groups
-// of rank v), base[r] = tickets before rank r; cell k, at place start[gc] +
-// gw[k] of every rank below gc, gets glist[base[r] + start[gc] + gw[k]] =
-// (k, r).  Writes the group count to *n_groups.
-constexpr int kGroupLds = 6144;    // start / base entries k_group_order keeps in LDS
+constexpr int kPSC = 48;                    // channels per workgroup
+constexpr int kPSTileWaves = 8;             // waves 0..7: tiles (two per SIMD)
+constexpr int kPSTeam = 3;                  // waves 8..10: rows of the even groups, 11..13: odd
+constexpr int kPSScanWaves = 2 * kPSTeam;
+constexpr int kPSDeal = kPSTileWaves + kPSScanWaves;         // wave 14: deals groups
+constexpr int kPSChain = kPSDeal + 1;                        // wave 15: start states
+constexpr int kPSThreads = 64 * (kPSChain + 1);
+constexpr int kPSSub = 64 * kPSTeam / kPSC;                  // row blocks of the scan
+constexpr int kPSRows = kGP / kPSSub;                        // rows of a thread
+constexpr int kPSStride = 2 * kPSC + 4;     // LDS row [v | sigmoid(g)]: 16 rows on 16 bank groups
+constexpr int kPSTiles = kPatch + (kGP - kPatch) / 16;       // most tiles of a group
+constexpr int kPSMask = (kGP + 63) / 64;    // 64-pair blocks of a group
+constexpr int kPSSlots = 4;                 // groups in flight in a workgroup
+static_assert(kPSSub * kPSC == 64 * kPSTeam && kGP % kPSSub == 0 && kPSRows < 64 &&
+                  kGP < 256 && 2 * kGW <= kGP, "group shape");
 
-__global__ void __launch_bounds__(kScanThreads)
-k_group_order(int nk, int nv, int sg, const int* __restrict__ pst, const int* __restrict__ pen,
-              const int* __restrict__ ghist, const int* __restrict__ gw, int* __restrict__ gstart,
-              int* __restrict__ gbase, int2* __restrict__ glist, int* __restrict__ n_groups) {
-    __shared__ int lds[2 * (kScanThreads / 64)];
-    __shared__ int sst[kGroupLds], sba[kGroupLds];
-    const bool inl = nv <= kGroupLds;      // else the tables are read from global memory
-    int carry = 0;
-    for (int r0 = 0; r0 < nv; r0 += kScanRound) {        // start: scan of ghist from the top
-        const int i0 = r0 + (int)threadIdx.x * kScanPer;
-        int v[kScanPer], sum = 0;
-        #pragma unroll
-        for (int q = 0; q < kScanPer; ++q) {
-            v[q] = i0 + q < nv ? ghist[nv - 1 - (i0 + q)] : 0;
-            sum += v[q];
-        }
-        int total;
-        int run = carry + block_exscan(sum, lds, &total);
-        carry += total;
-        #pragma unroll
-        for (int q = 0; q < kScanPer; ++q) {
-            const int i = nv - 1 - (i0 + q);
-            if (i0 + q < nv) {
-                gstart[i] = run;
-                if (inl) sst[i] = run;
-            }
-            run += v[q];
-        }
-    }
-    __syncthreads();
-    carry = 0;
-    for (int r0 = 0; r0 < nv; r0 += kScanRound) {        // base: prefix of start
-        const int i0 = r0 + (int)threadIdx.x * kScanPer;
-        int v[kScanPer], sum = 0;
-        #pragma unroll
-        for (int q = 0; q < kScanPer; ++q) {
-            v[q] = i0 + q < nv ? (inl ? sst[i0 + q] : gstart[i0 + q]) : 0;
-            sum += v[q];
-        }
-        int total;
-        int run = carry + block_exscan(sum, lds, &total);
-        carry += total;
-        #pragma unroll
-        for (int q = 0; q < kScanPer; ++q) {
-            if (i0 + q < nv) {
-                gbase[i0 + q] = run;
-                if (inl) sba[i0 + q] = run;
-            }
-            run += v[q];
-        }
-    }
-    if (threadIdx.x == 0) *n_groups = carry;
-    __syncthreads();
-    const int* st = inl ? sst : gstart;
-    const int* ba = inl ? sba : gbase;
-    for (int k = threadIdx.x; k < nk; k += kScanThreads) {
-        const int nc = (pen[k] - pst[k] + kCH - 1) / kCH, gc = (nc + sg - 1) / sg;
-        if (gc == 0) continue;
-        const int p = st[gc] + gw[k];
-        for (int r = 0; r < gc; ++r) glist[ba[r] + p] = make_int2(k, r);
-    }
+// One group on its way through a workgroup.
+struct PsSlot {
+    float* srow[kGP];               // state row of a pair's cell (groups with a cell end)
+    unsigned long long mfirst[kPSMask], mlast[kPSMask], mneed[kPSMask];
+    int ids[kGP];                   // 9 record + delta
+    unsigned char tsl[kPSTiles * 16], tdel[kPSTiles];   // pairs and delta of each tile
+    int ntiles, n, flags, word, r, slab;
+    int taken;                      // tiles taken
+    // arrivals over all groups that had the slot (a wave reaches the slot's next
+    // group only after all have passed this one): tile waves that have left the
+    // group, scan waves that have read T, written their maps and replayed
+    int left, read, mapped, replayed;
+};
+
+// kPSRows bits from bit i of a mask of kPSMask words
+__device__ __forceinline__ unsigned long long mask_window(const unsigned long long* m, int i) {
+    const int w = i >> 6, o = i & 63;
+    unsigned long long x = m[w] >> o;
+    if (o > 64 - kPSRows && w + 1 < kPSMask) x |= m[w + 1] << (64 - o);
+    return x & ((1ull << kPSRows) - 1ull);
 }
 
-template <int OUT, int HS, int SG>
-__global__ void __launch_bounds__(SG * ((OUT + 63) / 64) * 64)
-__attribute__((amdgpu_waves_per_eu(3, 8)))
-k_scan(const int* __restrict__ n_groups, int* __restrict__ ticket, unsigned tag,
-       const int2* __restrict__ glist, const int* __restrict__ cbeg, const int* __restrict__ cend,
-       const int* __restrict__ coff, const int* __restrict__ pst, const int* __restrict__ pen, int C,
-       const BlockDesc* __restrict__ bd, int li, const unsigned char* __restrict__ pair_need,
-       const float* __restrict__ QVG, float* __restrict__ Hout, unsigned long long* __restrict__ sw,
-       int* __restrict__ err, unsigned long long wait_ticks) {
-    constexpr int WPC = (OUT + 63) / 64;          // waves per chunk (64 channels each)
-    constexpr int NC = 2 * OUT;
-    __shared__ int stk;
-    __shared__ float sA[SG][OUT], sB[SG][OUT], sH[SG][OUT];
-    const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-    const int m = w / WPC;                        // the wave's chunk in the group
-    const int c = (w % WPC) * 64 + lane;          // the lane's channel
-    const bool on = c < OUT;
-    const int cc = on ? c : 0;
-    if (t == 0) stk = atomicAdd(ticket, 1);
+// Hand-over between a workgroup's waves by counters in LDS: what a wave wrote
+// to LDS before it arrives is seen by a wave that waited for the count.
+__device__ __forceinline__ int lds_get(const int* p) {
+    return __builtin_amdgcn_readfirstlane(
+        __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+}
+__device__ __forceinline__ void lds_arrive(int* p) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    if ((threadIdx.x & 63) == 0)
+        __hip_atomic_fetch_add(p, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void lds_wait(const int* p, int v) {
+    while (lds_get(p) < v) __builtin_amdgcn_s_sleep(1);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+template <int IN, int OUT, bool ALL, bool NT>
+__global__ void __launch_bounds__(kPSThreads, 4)
+k_pscan(const int* __restrict__ n_groups, int* __restrict__ ticket, unsigned tag,
+        const int4* __restrict__ glist, const uint2* __restrict__ pent, const float* __restrict__ X,
+        const float* __restrict__ pp, int C, const BlockDesc* __restrict__ bd, int li,
+        float* __restrict__ Hout, unsigned long long* __restrict__ sw, int* __restrict__ err,
+        unsigned long long wait_ticks) {
+    using P = ProjPackT<IN, OUT>;
+    constexpr int KG = P::KG, NS = OUT / kPSC, NJ = 2 * kPSC / 16;
+    __shared__ __align__(16) float T[2][(kGP + 1) * kPSStride];   // row kGP: the spare row
+    __shared__ PsSlot slot[kPSSlots];
+    __shared__ float sA[2][kPSSub][kPSC], sB[2][kPSSub][kPSC];    // sA: then the start states
+    __shared__ int dcnt[kPatch];
+    // groups dealt, the workgroup's groups (once known), groups with start states
+    __shared__ int dealt, n_mine, starts;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (threadIdx.x == 0) {
+        dealt = starts = 0;
+        n_mine = 0x7fffffff;
+    }
+    if (threadIdx.x < kPSSlots) {
+        PsSlot& S = slot[threadIdx.x];
+        S.left = S.read = S.mapped = S.replayed = 0;
+    }
     __syncthreads();
-    const int gi = stk;
-    if (gi >= *n_groups) return;                  // uniform over the workgroup
-    const int2 kr = glist[gi];
-    const int k = kr.x, r = kr.y;
-    const int nc = (pen[k] - pst[k] + kCH - 1) / kCH;
-    const int slot0 = coff[k];                    // the cell's first chunk
-    const int c0 = slot0 + r * SG;               // the group's first chunk
-    const int ng = min(SG, nc - r * SG);
-    const bool have = m < ng;
-    int s = 0, n = 0;
-    float sg[kCH], vv[kCH];
-    if (have) {
-        s = cbeg[c0 + m];
-        n = cend[c0 + m] - s;
-        // all kCH rows, eight from one base address (their offsets fit the
-        // load's immediate field; a clamped index per row cost a 64-bit
-        // address register per load).  Rows past the chunk's end stay inside
-        // the row buffer (kCH rows of padding past the largest row count) and
-        // are not used.
-        const float* row = QVG + (size_t)s * NC + cc;
-        #pragma unroll
-        for (int q8 = 0; q8 < kCH; q8 += 8) {
-            const float* rb = row + (size_t)q8 * NC;
+    // arrivals of all `waves` in group g's slot, up to and with group g
+    auto count = [](int waves, int g) { return waves * (g / kPSSlots + 1); };
+    // waits for group g to be dealt; false: the workgroup has no such group
+    auto have_group = [&](int g) {
+        for (;;) {
+            if (lds_get(&dealt) > g) break;
+            if (lds_get(&n_mine) <= g) return false;
+            __builtin_amdgcn_s_sleep(1);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        return true;
+    };
+
+    // the few instructions of the other waves go ahead of the tiles' streams
+    if (wv >= kPSDeal) __builtin_amdgcn_s_setprio(3);
+    else if (wv >= kPSTileWaves) __builtin_amdgcn_s_setprio(2);
+    if (wv < kPSTileWaves) {
+        // ---- tiles: v, sigmoid(g) of 16 pairs of one delta --------------------
+        // weights are loaded one float4 group (a part, four k-steps) at a time,
+        // DW - 1 parts ahead, and the next tile's input rows while a tile runs
+        constexpr int NQ = NJ * KG, DW = KG == 2 ? 4 : 6;
+        static_assert(NQ % DW == 0 && NQ >= 8, "weight ring");
+        const int lc = lane & 15, lk = lane >> 4;
+        f32x4 xb[KG], xn[KG], wb[DW];
+        auto load_x = [&](int id, f32x4 (&x)[KG]) {
+            const float* xp = X + (size_t)((unsigned)id / (unsigned)kPatch) * IN;
             #pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                vv[q8 + q] = __builtin_nontemporal_load(rb + q * NC);
-                sg[q8 + q] = __builtin_nontemporal_load(rb + q * NC + OUT);
+            for (int g = 0; g < KG; ++g) {
+                if (P::steps(g) == 4) {
+                    x[g] = *(const SSLA_GLOBAL f32x4*)(xp + P::kidx(g, lk, 0));
+                } else {
+                    const f32x2 v = *(const SSLA_GLOBAL f32x2*)(xp + P::kidx(g, lk, 0));
+                    x[g] = f32x4{v[0], v[1], 0.f, 0.f};
+                }
+            }
+        };
+        // part q of a tile: group q % KG of item q / KG (ds = delta, slab)
+        auto load_w = [&](int ds, int q, f32x4& w) {
+            const SSLA_GLOBAL f32x4* src = (const SSLA_GLOBAL f32x4*)pp + (size_t)(ds * NQ + q) * 64;
+            if (P::steps(q % KG) == 4) {
+                w = src[(unsigned)lane];
+            } else {
+                const f32x2 v = *(const SSLA_GLOBAL f32x2*)(src + (unsigned)lane);
+                w = f32x4{v[0], v[1], 0.f, 0.f};
+            }
+        };
+        auto take = [&](PsSlot& S) { return lane == 0 ? atomicAdd(&S.taken, 1) : 0; };
+        for (int g = 0; have_group(g);) {
+            PsSlot* S = &slot[g % kPSSlots];
+            int nt = __builtin_amdgcn_readfirstlane(S->ntiles);
+            int tile = __builtin_amdgcn_readfirstlane(take(*S));
+            if (tile >= nt) {
+                lds_arrive(&S->left);
+                ++g;
+                continue;
+            }
+            int lp = S->tsl[tile * 16 + lc];
+            int ds = __builtin_amdgcn_readfirstlane(S->tdel[tile] * NS + S->slab);
+            load_x(S->ids[lp < kGP ? lp : 0], xb);
+            #pragma unroll
+            for (int q = 0; q < DW - 1; ++q) load_w(ds, q, wb[q]);
+            for (;;) {
+                // T[g % 2] is free once group g - 2 has been read
+                if (g > 1) lds_wait(&slot[(g - 2) % kPSSlots].read, count(kPSTeam, g - 2));
+                float* row = &T[g & 1][lp * kPSStride + 4 * lk];
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                // the next tile, of this group or, if it is dealt, the next one
+                // (none: this tile again, so that the loads carry no branch);
+                // its look-ups are spread over the first parts
+                PsSlot* SN = S;
+                int tn = 0, lpn = 0, idn = 0, dsn = 0, gn = g;
+                bool more = true;
+                #pragma unroll
+                for (int q = 0; q < NQ; ++q) {
+                    const int j = q / KG, kg = q % KG;
+                    if (q == 0) tn = take(*S);
+                    if (q == 1) {
+                        tn = __builtin_amdgcn_readfirstlane(tn);
+                        if (tn >= nt) {
+                            gn = g + 1;
+                            more = lds_get(&dealt) > gn;
+                            if (more) {
+                                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                                SN = &slot[gn % kPSSlots];
+                                tn = __builtin_amdgcn_readfirstlane(take(*SN));
+                                more = tn < __builtin_amdgcn_readfirstlane(SN->ntiles);
+                            }
+                            if (!more) tn = 0;
+                        }
+                        lpn = SN->tsl[tn * 16 + lc];
+                        dsn = SN->tdel[tn] * NS + SN->slab;
+                    }
+                    if (q == 2) idn = SN->ids[lpn < kGP ? lpn : 0];
+                    if (q == 3) load_x(idn, xn);
+                    if (q == NQ - DW + 1) dsn = __builtin_amdgcn_readfirstlane(dsn);
+                    if (q + DW - 1 < NQ) load_w(ds, q + DW - 1, wb[(q + DW - 1) % DW]);
+                    else load_w(dsn, q + DW - 1 - NQ, wb[(q + DW - 1) % DW]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (kg == 0) acc = f32x4{0.f, 0.f, 0.f, 0.f};
+                    #pragma unroll
+                    for (int i = 0; i < P::steps(kg); ++i)
+                        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wb[q % DW][i], xb[kg][i], acc, 0, 0, 0);
+                    if (kg == KG - 1) {
+                        if (j >= NJ / 2) {
+                            #pragma unroll
+                            for (int i = 0; i < 4; ++i) acc[i] = sigmoid_fast(acc[i]);
+                        }
+                        *reinterpret_cast<f32x4*>(row + 16 * j) = acc;
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (gn != g) {
+                    lds_arrive(&S->left);
+                    g = gn;
+                    if (!more) {
+                        // (a tile counter taken past its end is harmless)
+                        break;
+                    }
+                    S = SN;
+                    nt = __builtin_amdgcn_readfirstlane(S->ntiles);
+                }
+                lp = lpn;
+                ds = dsn;
+                #pragma unroll
+                for (int k = 0; k < KG; ++k) xb[k] = xn[k];
             }
         }
-        float A = 1.f, B = 0.f;
-        #pragma unroll
-        for (int q = 0; q < kCH; ++q) {
-            sg[q] = sigmoid_fast(sg[q]);
-            if (q < n) {
-                A *= sg[q];
-                B = fmaf(sg[q], B, vv[q]);
+    } else if (wv < kPSDeal) {
+        // ---- rows: maps, replay (two teams, every other group each) --------------
+        const int team = (wv - kPSTileWaves) / kPSTeam;
+        const int ct = (int)threadIdx.x - 64 * (kPSTileWaves + team * kPSTeam);
+        const int sub = ct / kPSC, ch = ct - sub * kPSC, i0 = sub * kPSRows;
+        for (int g = team; have_group(g); g += 2) {
+            PsSlot& S = slot[g % kPSSlots];
+            float vv[kPSRows], ss[kPSRows];
+            lds_wait(&S.left, count(kPSTileWaves, g));
+            const float* row = &T[g & 1][i0 * kPSStride + ch];
+            #pragma unroll
+            for (int q = 0; q < kPSRows; ++q) {
+                vv[q] = row[q * kPSStride];
+                ss[q] = row[q * kPSStride + kPSC];
             }
-        }
-        if (on) {
-            sA[m][c] = A;
-            sB[m][c] = B;
-        }
-    }
-    __syncthreads();
-    if (w < WPC) {                                // the first chunk's waves chain the group
-        const bool last = (r + 1) * SG >= nc;    // the cell's last group
-        float* hp0 = bd[k / C].hidden[li] + (size_t)(k % C) * OUT + cc;
-        unsigned long long* P = sw + (size_t)c0 * 3 * OUT + cc;
-        float SA = 1.f, SB = 0.f;
-        for (int q = 0; q < ng; ++q) {
-            SB = fmaf(sA[q][cc], SB, sB[q][cc]);
-            SA *= sA[q][cc];
-        }
-        float h0;
-        if (r == 0) {
-            h0 = on ? *hp0 : 0.f;
-        } else {
-            if (!last && on) {
-                sw_put(P + OUT, SA, tag);
-                sw_put(P + 2 * OUT, SB, tag);
+            lds_arrive(&S.read);
+            const int n = __builtin_amdgcn_readfirstlane(S.n);
+            const int flags = __builtin_amdgcn_readfirstlane(S.flags);
+            if (n < kGP) {
+                // rows past the group's pairs leave a state as it is
+                #pragma unroll
+                for (int q = 0; q < kPSRows; ++q) {
+                    vv[q] = i0 + q < n ? vv[q] : 0.f;
+                    ss[q] = i0 + q < n ? ss[q] : 1.f;
+                }
             }
-            h0 = scan_lookback<OUT, SG>(sw, slot0, r, cc, on, tag,
-                                    (unsigned long long)wall_clock64() + wait_ticks, err);
-        }
-        if (on) {
-            const float hend = fmaf(SA, h0, SB);
-            if (last) *hp0 = hend;
-            else sw_put(P, hend, tag);
-        }
-        float h = h0;
-        for (int q = 0; q < ng; ++q) {
-            if (on) sH[q][c] = h;
-            h = fmaf(sA[q][cc], h, sB[q][cc]);
-        }
-    }
-    __syncthreads();
-    if (!have) return;
-    // replay from the chunk's start state; lane l reads pair s + l's need flag
-    const unsigned long long use =
-        __ballot(lane < n && (!pair_need || pair_need[s + lane]));
-    float h = on ? sH[m][c] : 0.f;
-    float* hp = Hout + (size_t)s * HS + cc;
-    #pragma unroll
-    for (int q = 0; q < kCH; ++q) {
-        if (q < n) {
-            h = fmaf(sg[q], h, vv[q]);
-            if (on && ((use >> q) & 1ull)) {
-                // the compact h rows (L4, L5) go out nontemporal: the
-                // contraction that gathers them next runs faster (L4 179 ->
-                // 160 us for +9 us here); L6's in-place rows lose by it
-                if constexpr (HS == OUT) __builtin_nontemporal_store(h, hp + (size_t)q * HS);
-                else gstore(hp + (size_t)q * HS, h);
+            if (flags & kGStart) {
+                const unsigned long long fw = mask_window(S.mfirst, i0);
+                #pragma unroll
+                for (int q = 0; q < kPSRows; ++q)
+                    if ((fw >> q) & 1u) {
+                        vv[q] = fmaf(ss[q], gload(S.srow[i0 + q] + ch), vv[q]);
+                        ss[q] = 0.f;
+                    }
             }
+            float A = 1.f, B = 0.f;
+            #pragma unroll
+            for (int q = 0; q < kPSRows; ++q) {
+                A *= ss[q];
+                B = fmaf(ss[q], B, vv[q]);
+            }
+            sA[g & 1][sub][ch] = A;
+            sB[g & 1][sub][ch] = B;
+            lds_arrive(&S.mapped);
+            lds_wait(&starts, g + 1);
+            float h = sA[g & 1][sub][ch];
+            #pragma unroll
+            for (int q = 0; q < kPSRows; ++q) {
+                h = fmaf(ss[q], h, vv[q]);
+                vv[q] = h;
+            }
+            float* const hb = Hout + __builtin_amdgcn_readfirstlane(S.slab) * kPSC + ch;
+            auto put = [&](int q) {
+                float* hp = hb + (size_t)(unsigned)S.ids[i0 + q] * OUT;
+                if constexpr (NT) __builtin_nontemporal_store(vv[q], (SSLA_GLOBAL float*)hp);
+                else gstore(hp, vv[q]);
+            };
+            if (ALL && n == kGP) {
+                #pragma unroll
+                for (int q = 0; q < kPSRows; ++q) put(q);
+            } else {
+                const unsigned long long nw =
+                    ALL ? (1ull << max(0, min(kPSRows, n - i0))) - 1ull : mask_window(S.mneed, i0);
+                #pragma unroll
+                for (int q = 0; q < kPSRows; ++q)
+                    if ((nw >> q) & 1u) put(q);
+            }
+            if (flags & kGEnd) {
+                const unsigned long long lw = mask_window(S.mlast, i0);
+                #pragma unroll
+                for (int q = 0; q < kPSRows; ++q)
+                    if ((lw >> q) & 1u) gstore(S.srow[i0 + q] + ch, vv[q]);
+            }
+            lds_arrive(&S.replayed);
+        }
+    } else if (wv == kPSDeal) {
+        // ---- deals the pairs of the next groups into tiles of one delta -----------
+        const int total = *n_groups * NS;
+        auto draw = [&]() { return lane == 0 ? atomicAdd(ticket, 1) : 0; };
+        auto fetch = [&](int tk) { return tk < total ? glist[tk / NS] : make_int4(0, 0, 0, 0); };
+        uint2 e[kPSMask];
+        auto load_pairs = [&](int4 gd) {
+            const int n = gd.y & 0xffff;
+            #pragma unroll
+            for (int j = 0; j < kPSMask; ++j) {
+                e[j] = make_uint2(0u, 0u);
+                if (64 * j + lane < n) e[j] = pent[gd.x + 64 * j + lane];
+            }
+        };
+        // in flight: the next group's pairs, the group after it, the ticket after that
+        int tk = __builtin_amdgcn_readfirstlane(draw()), tk1 = __builtin_amdgcn_readfirstlane(draw());
+        int tk2 = draw();
+        int4 gd = fetch(tk), gd1 = fetch(tk1);
+        load_pairs(gd);
+        for (int g = 0;; ++g) {
+            if (tk >= total) {
+                if (lane == 0) __hip_atomic_store(&n_mine, g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                break;
+            }
+            uint2 ec[kPSMask];
+            #pragma unroll
+            for (int j = 0; j < kPSMask; ++j) ec[j] = e[j];
+            load_pairs(gd1);
+            const int t2 = __builtin_amdgcn_readfirstlane(tk2);
+            const int4 gd2 = fetch(t2);
+            tk2 = draw();
+            // the slot is free once group g - kPSSlots has been replayed
+            PsSlot& S = slot[g % kPSSlots];
+            if (g >= kPSSlots) lds_wait(&S.replayed, count(kPSTeam, g - kPSSlots));
+            const int flags = __builtin_amdgcn_readfirstlane(gd.y), n = flags & 0xffff;
+            const int slab = NS == 1 ? 0 : tk % NS;
+            if (lane < kPatch) dcnt[lane] = 0;
+            for (int i = lane; i < kPSTiles * 16 / 4; i += 64)
+                reinterpret_cast<int*>(S.tsl)[i] = kGP * 0x01010101;
+            int rank[kPSMask], delta[kPSMask];
+            #pragma unroll
+            for (int j = 0; j < kPSMask; ++j) {
+                const bool on = 64 * j + lane < n;
+                delta[j] = (int)((ec[j].x & ~kPairNeed) % (unsigned)kPatch);
+                rank[j] = on ? atomicAdd(&dcnt[delta[j]], 1) : 0;
+            }
+            // a cell's first and last pairs
+            #pragma unroll
+            for (int j = 0; j < kPSMask; ++j) {
+                const int i = 64 * j + lane;
+                bool first = false, last = false;
+                if (flags & kGMulti) {
+                    uint32_t up = (uint32_t)__shfl_up((int)ec[j].y, 1);
+                    uint32_t dn = (uint32_t)__shfl_down((int)ec[j].y, 1);
+                    const uint32_t pe = (uint32_t)__builtin_amdgcn_readlane((int)ec[j ? j - 1 : 0].y, 63);
+                    const uint32_t ns = (uint32_t)__builtin_amdgcn_readlane(
+                        (int)ec[j + 1 < kPSMask ? j + 1 : j].y, 0);
+                    if (lane == 0) up = pe;
+                    if (lane == 63) dn = ns;
+                    first = up != ec[j].y;
+                    last = dn != ec[j].y;
+                }
+                const unsigned long long mf = __ballot(i < n && (i == 0 ? (flags & kGStart) != 0 : first));
+                const unsigned long long ml = __ballot(i < n && (i == n - 1 ? (flags & kGEnd) != 0 : last));
+                const unsigned long long mn = __ballot(i < n && (ec[j].x & kPairNeed));
+                if (lane == 0) {
+                    S.mfirst[j] = mf;
+                    S.mlast[j] = ml;
+                    S.mneed[j] = mn;
+                }
+            }
+            int base[kPSMask] = {}, nt = 0;
+            #pragma unroll
+            for (int d = 0; d < kPatch; ++d) {
+                #pragma unroll
+                for (int j = 0; j < kPSMask; ++j)
+                    if (delta[j] == d) base[j] = nt;
+                nt += (dcnt[d] + 15) >> 4;
+            }
+            #pragma unroll
+            for (int j = 0; j < kPSMask; ++j) {
+                const int i = 64 * j + lane;
+                if (i < n) {
+                    S.tsl[base[j] * 16 + rank[j]] = (unsigned char)i;
+                    if ((rank[j] & 15) == 0) S.tdel[base[j] + (rank[j] >> 4)] = (unsigned char)delta[j];
+                    S.ids[i] = (int)(ec[j].x & ~kPairNeed);
+                    if (flags & (kGStart | kGEnd)) {
+                        const int k = (int)ec[j].y, b = k / C;
+                        S.srow[i] = bd[b].hidden[li] + (size_t)(k - b * C) * OUT + slab * kPSC;
+                    }
+                }
+            }
+            if (lane == 0) {
+                S.ntiles = nt;
+                S.n = n;
+                S.flags = flags;
+                S.word = gd.z;
+                S.r = gd.w;
+                S.slab = slab;
+                S.taken = 0;
+            }
+            lds_arrive(&dealt);
+            tk = tk1;
+            tk1 = t2;
+            gd = gd1;
+            gd1 = gd2;
+        }
+    } else {
+        // ---- the groups' maps and start states -----------------------------------
+        const bool con = lane < kPSC;
+        const int cl = con ? lane : 0;
+        for (int g = 0; have_group(g); ++g) {
+            const PsSlot& S = slot[g % kPSSlots];
+            lds_wait(&S.mapped, count(kPSTeam, g));
+            const int flags = __builtin_amdgcn_readfirstlane(S.flags);
+            const int word = __builtin_amdgcn_readfirstlane(S.word);
+            const int r = __builtin_amdgcn_readfirstlane(S.r);
+            const int cc = __builtin_amdgcn_readfirstlane(S.slab) * kPSC + cl;
+            float a[kPSSub], b[kPSSub], SA = 1.f, SB = 0.f;
+            #pragma unroll
+            for (int q = 0; q < kPSSub; ++q) {
+                a[q] = sA[g & 1][q][cl];
+                b[q] = sB[g & 1][q][cl];
+            }
+            #pragma unroll
+            for (int q = 0; q < kPSSub; ++q) {
+                SB = fmaf(a[q], SB, b[q]);
+                SA *= a[q];
+            }
+            unsigned long long* W = sw + (size_t)word * 3 * OUT + cc;
+            float h = 0.f;
+            if (flags & kGStart) {
+                if (!(flags & kGEnd) && con) sw_put(W, SB, tag);       // SA = 0: no start state
+            } else {
+                if (!(flags & kGEnd) && con) {
+                    sw_put(W + OUT, SA, tag);
+                    sw_put(W + 2 * OUT, SB, tag);
+                }
+                h = scan_lookback<OUT>(sw, word - r, r, cc, con, tag,
+                                       (unsigned long long)wall_clock64() + wait_ticks, err);
+                if (!(flags & kGEnd) && con) sw_put(W, fmaf(SA, h, SB), tag);
+            }
+            #pragma unroll
+            for (int q = 0; q < kPSSub; ++q) {
+                if (con) sA[g & 1][q][cl] = h;
+                h = fmaf(a[q], h, b[q]);
+            }
+            lds_arrive(&starts);
         }
     }
 }
@@ -1468,7 +1663,8 @@ k_scan(const int* __restrict__ n_groups, int* __restrict__ ticket, unsigned tag,
 // values of the goW steps.  The weights stream from the L2 (shared by all
 // waves) one (delta, channel tile) item ahead.  LayerNorm in fp64 over the
 // four lanes that hold a record's outputs (ds_swizzle and ds_bpermute sums).
-// HR rows are HS floats apart (the scan's h output rows).
+// HR holds the h row of pair (record g, delta d) at 9 g + d; whether the pair
+// exists follows from g's centre cell (s2 coordinates >> shift, on a W x H grid).
 // WPS asks the compiler for at least that many waves per SIMD; with the
 // unrolled item loop L4 (RT = 2) compiles to 120 registers, 4 waves per SIMD.
 // ---------------------------------------------------------------------------
@@ -1500,10 +1696,11 @@ __device__ __forceinline__ double sum4_lanes(double v, int lane) {
 constexpr int kOutKS5 = 3, kOutKS6 = 3, kOutKS7 = 3;
 constexpr int kOutRT5 = 1, kOutRT6 = 1, kOutRT7 = 1;
 
-template <int IN, int OUT, int RT, int KS, int WPS = 1, int HS = 2 * OUT>
+template <int IN, int OUT, int RT, int KS, int WPS = 1>
 __global__ void __launch_bounds__(64 * KS, WPS)
 k_outt(int n_max, const int* __restrict__ n_dev, const int* __restrict__ list,
-       const float* __restrict__ X, const int* __restrict__ pos, const float* __restrict__ HR,
+       const float* __restrict__ X, const int* __restrict__ cell2, int shift, int W2, int W, int H,
+       const float* __restrict__ HR,
        const float* __restrict__ po, const float* __restrict__ gamma,
        const float* __restrict__ beta, float* __restrict__ Y) {
     using O = OutPackT<IN, OUT>;
@@ -1519,7 +1716,9 @@ k_outt(int n_max, const int* __restrict__ n_dev, const int* __restrict__ list,
         const int r = t / kPatch, d = t - r * kPatch;
         const int q = base + r;
         const int rr = q < n ? (list ? list[q] : q) : -1;
-        sp[r][d] = rr >= 0 ? pos[(size_t)rr * kPatch + d] : -1;
+        const int cell = rr >= 0 ? cell2[rr] : -1;
+        const int tx = ((cell % W2) >> shift) + 1 - d % 3, ty = ((cell / W2) >> shift) + 1 - d / 3;
+        sp[r][d] = cell >= 0 && tx >= 0 && tx < W && ty >= 0 && ty < H ? rr * kPatch + d : -1;
     }
     int rec[RT];
     #pragma unroll
@@ -1578,7 +1777,7 @@ k_outt(int n_max, const int* __restrict__ n_dev, const int* __restrict__ list,
         for (int rt = 0; rt < RT; ++rt) {
             const int p = sp[16 * rt + j][d];
             pv[rt] = p;
-            hv[rt] = *(const SSLA_GLOBAL f32x4*)(HR + (size_t)(p < 0 ? 0 : p) * HS + 16 * ct + 4 * g);
+            hv[rt] = *(const SSLA_GLOBAL f32x4*)(HR + (size_t)(p < 0 ? 0 : p) * OUT + 16 * ct + 4 * g);
         }
     };
     auto compute = [&](const f32x4 (&aq)[KG], const f32x4 (&ag)[NT], const f32x4 (&hv)[RT],
@@ -1923,25 +2122,22 @@ struct Workspace {
     int cap_keys = 0;
     void* base = nullptr;
     size_t bytes = 0;
-    float *X0, *X1, *X2, *X3, *X4, *QVG, *H7;
-    int *cell2, *pos2, *pos3, *list2, *list3, *counts;
-    int *st2, *en2, *st3, *en3, *pst2, *pen2, *pst3, *pen3, *last3, *cnt3;
-    unsigned char *pneed2, *pneed3;            // per sorted pair: its record needs the output
-    int *coff2, *coff3;                        // first chunk of every key
-    int *ckey2, *cbeg2, *cend2, *ckey3, *cbeg3, *cend3;
+    float *X0, *X1, *X2, *X3, *X4, *HR, *H7;   // HR: h rows of one layer, row 9 record + delta
+    int *cell2, *list2, *list3, *counts;
+    int *st2, *en2, *st3, *en3, *pst2, *pst3, *pcnt, *last3, *cnt3;
+    uint2 *pent2, *pent3;                      // per sorted pair: {9 record + delta | need, cell key}
+    int *goff2, *goff3;                        // first published-word slot of every key
     int *sidx;                                 // sorted s2 position of every record
     int *n2, *t3, *n3;                         // pass-2 records per s2 / s3 key, pass-3 per s3 key
     int *off2, *off3;                          // first pass-2 / pass-3 list slot of every key
     int *bh;                                   // radix-sort tile histograms
     unsigned char* old2;                       // s2 counters before the call
-    unsigned long long* sw;                    // one-pass scan: published words, per group's first chunk
-    int *ghist, *gw, *gstart, *gbase;          // one-pass scan: s2 group order tables
-    int2* glist;                               // one-pass scan: (cell, rank) of every s2 ticket
-    int *ghist3, *gw3, *gstart3, *gbase3;      // ... and of the s3 level
-    int2* glist3;
-    int nv = 0;                                // entries of ghist / gstart / gbase
-    int* scan_err = nullptr;                   // host memory: a one-pass scan wait ran out
-    float* trash;                              // sink of the projection's absent rows
+    unsigned long long* sw;                    // k_pscan: published words, per group
+    int *ghist, *gw, *gcnt, *gend, *gstart, *gbase;          // s2 group order tables
+    int4* glist;                                             // group of every s2 ticket
+    int *ghist3, *gw3, *gcnt3, *gend3, *gstart3, *gbase3;    // ... and of the s3 level
+    int4* glist3;
+    int* scan_err = nullptr;                   // host memory: a look-back wait ran out
     unsigned char *owner, *pass2, *pass3;
     uint32_t *ka, *kb, *va, *vb, *key3g;
     BlockDesc* bd;
@@ -1950,7 +2146,6 @@ struct Workspace {
     hipEvent_t s2_ordered = nullptr;   // s2 tables and pass2 are complete
     hipEvent_t s3_ordered = nullptr;   // s3 tables and pass3 are complete
     hipEvent_t side_done = nullptr;    // the side stream's last work of a call
-    hipEvent_t s2_groups = nullptr;    // the one-pass scan's group order is built
     int bh_ints = 0;
     int cus = 0;                       // compute units of the device
     int clk_khz = 0;                   // wall-clock (s_memrealtime) rate
@@ -1995,7 +2190,7 @@ int flush_pending(Workspace& w, size_t n) {
 
 std::mutex g_ws_mu;
 Workspace g_ws;
-unsigned g_scan_tag = 0;     // tag of the one-pass scan's last launch (under g_ws_mu)
+unsigned g_scan_tag = 0;     // tag of k_pscan's last launch (under g_ws_mu)
 
 #define HIPCHK(call)                                                          \
     do {                                                                      \
@@ -2021,10 +2216,12 @@ int ensure_workspace(int E, int nkeys) {
     const int cap = std::max(E, std::max(g_ws.cap, 1024));
     const int ck = std::max(nkeys, g_ws.cap_keys);
     const size_t P = (size_t)cap * kPatch;
-    const size_t mc = P / kCH + (size_t)ck + 1;    // chunk bound: full chunks + one tail per key
+    // group bound: full groups + one tail per key (shared groups are fewer
+    // than the keys in them)
+    const size_t mg = P / kGP + (size_t)ck + 1;
     // a cell's pairs come from distinct records: at most cap, so a cell has at
-    // most cap / (kCH kSG) + 2 groups of the one-pass scan
-    const size_t nv = (size_t)cap / (kCH * std::min(kSG, kSG3)) + 3;
+    // most cap / kGP + 1 groups
+    const size_t nv = (size_t)cap / kGP + 3;
     // radix-sort tile histograms: (1 << kRMaxBits) digits x tiles
     const size_t bh = ((size_t)1 << kRMaxBits) * (size_t)((cap + kRTile - 1) / kRTile);
     struct Item { void** dst; size_t bytes; };
@@ -2035,13 +2232,11 @@ int ensure_workspace(int E, int nkeys) {
         {(void**)&w.X2, sizeof(float) * (size_t)cap * SSLA_C2},
         {(void**)&w.X3, sizeof(float) * (size_t)cap * SSLA_C3},
         {(void**)&w.X4, sizeof(float) * (size_t)cap * SSLA_C3},
-        // [v | g] rows, and kCH rows of padding that a scan chunk may read past
-        // the last one
-        {(void**)&w.QVG, sizeof(float) * (P + kCH) * 2 * SSLA_C3},
+        {(void**)&w.HR, sizeof(float) * P * SSLA_C3},
         {(void**)&w.H7, sizeof(float) * (size_t)cap * 7},
         {(void**)&w.cell2, sizeof(int) * (size_t)cap},
-        {(void**)&w.pos2, sizeof(int) * P},
-        {(void**)&w.pos3, sizeof(int) * P},
+        {(void**)&w.pent2, sizeof(uint2) * P},
+        {(void**)&w.pent3, sizeof(uint2) * P},
         {(void**)&w.list2, sizeof(int) * (size_t)cap},
         {(void**)&w.list3, sizeof(int) * (size_t)cap},
         {(void**)&w.counts, sizeof(int) * 16},
@@ -2050,9 +2245,8 @@ int ensure_workspace(int E, int nkeys) {
         {(void**)&w.st3, sizeof(int) * (size_t)ck},
         {(void**)&w.en3, sizeof(int) * (size_t)ck},
         {(void**)&w.pst2, sizeof(int) * (size_t)ck},
-        {(void**)&w.pen2, sizeof(int) * (size_t)ck},
         {(void**)&w.pst3, sizeof(int) * (size_t)ck},
-        {(void**)&w.pen3, sizeof(int) * (size_t)ck},
+        {(void**)&w.pcnt, sizeof(int) * (size_t)ck},
         {(void**)&w.last3, sizeof(int) * (size_t)ck},
         {(void**)&w.cnt3, sizeof(int) * (size_t)ck},
         {(void**)&w.owner, (size_t)cap},
@@ -2063,11 +2257,9 @@ int ensure_workspace(int E, int nkeys) {
         {(void**)&w.va, sizeof(uint32_t) * (size_t)cap},
         {(void**)&w.vb, sizeof(uint32_t) * (size_t)cap},
         {(void**)&w.key3g, sizeof(uint32_t) * (size_t)cap},
-        {(void**)&w.pneed2, P},
-        {(void**)&w.pneed3, P},
         {(void**)&w.sidx, sizeof(int) * (size_t)cap},
-        {(void**)&w.coff2, sizeof(int) * (size_t)ck},
-        {(void**)&w.coff3, sizeof(int) * (size_t)ck},
+        {(void**)&w.goff2, sizeof(int) * (size_t)ck},
+        {(void**)&w.goff3, sizeof(int) * (size_t)ck},
         {(void**)&w.n2, sizeof(int) * (size_t)ck},
         {(void**)&w.t3, sizeof(int) * (size_t)ck},
         {(void**)&w.n3, sizeof(int) * (size_t)ck},
@@ -2075,24 +2267,21 @@ int ensure_workspace(int E, int nkeys) {
         {(void**)&w.off3, sizeof(int) * (size_t)ck},
         {(void**)&w.bh, sizeof(int) * bh},
         {(void**)&w.old2, (size_t)ck},
-        {(void**)&w.ckey2, sizeof(int) * mc},
-        {(void**)&w.cbeg2, sizeof(int) * mc},
-        {(void**)&w.cend2, sizeof(int) * mc},
-        {(void**)&w.ckey3, sizeof(int) * mc},
-        {(void**)&w.cbeg3, sizeof(int) * mc},
-        {(void**)&w.cend3, sizeof(int) * mc},
-        {(void**)&w.sw, sizeof(unsigned long long) * mc * 3 * SSLA_C3},
+        {(void**)&w.sw, sizeof(unsigned long long) * mg * 3 * SSLA_C3},
         {(void**)&w.ghist, sizeof(int) * nv},
         {(void**)&w.gstart, sizeof(int) * nv},
         {(void**)&w.gbase, sizeof(int) * nv},
         {(void**)&w.gw, sizeof(int) * (size_t)ck},
-        {(void**)&w.glist, sizeof(int2) * (mc / kSG + (size_t)ck + 1)},
+        {(void**)&w.gcnt, sizeof(int) * (size_t)ck},
+        {(void**)&w.gend, sizeof(int) * (size_t)ck},
+        {(void**)&w.glist, sizeof(int4) * mg},
         {(void**)&w.ghist3, sizeof(int) * nv},
         {(void**)&w.gstart3, sizeof(int) * nv},
         {(void**)&w.gbase3, sizeof(int) * nv},
         {(void**)&w.gw3, sizeof(int) * (size_t)ck},
-        {(void**)&w.glist3, sizeof(int2) * (mc / kSG3 + (size_t)ck + 1)},
-        {(void**)&w.trash, sizeof(float) * 4 * 64},
+        {(void**)&w.gcnt3, sizeof(int) * (size_t)ck},
+        {(void**)&w.gend3, sizeof(int) * (size_t)ck},
+        {(void**)&w.glist3, sizeof(int4) * mg},
         {(void**)&w.bd, sizeof(BlockDesc) * SSLA_MAX_BLOCKS},
     };
     size_t total = 0;
@@ -2105,8 +2294,7 @@ int ensure_workspace(int E, int nkeys) {
         p += align_up(it.bytes);
     }
     // no stale word may carry a future launch's tag
-    HIPCHK(hipMemset(w.sw, 0, sizeof(unsigned long long) * mc * 3 * SSLA_C3));
-    w.nv = (int)nv;
+    HIPCHK(hipMemset(w.sw, 0, sizeof(unsigned long long) * mg * 3 * SSLA_C3));
     if (!w.scan_err) {
         HIPCHK(hipHostMalloc((void**)&w.scan_err, sizeof(int), hipHostMallocCoherent));
         *w.scan_err = 0;
@@ -2116,7 +2304,6 @@ int ensure_workspace(int E, int nkeys) {
         HIPCHK(hipEventCreateWithFlags(&w.s2_ordered, hipEventDisableTiming));
         HIPCHK(hipEventCreateWithFlags(&w.s3_ordered, hipEventDisableTiming));
         HIPCHK(hipEventCreateWithFlags(&w.side_done, hipEventDisableTiming));
-        HIPCHK(hipEventCreateWithFlags(&w.s2_groups, hipEventDisableTiming));
         HIPCHK(hipStreamCreateWithFlags(&w.side, hipStreamNonBlocking));
         HIPCHK(hipMalloc(&w.packed, sizeof(float) * packed_weight_floats_d()));
         int dev = 0;
@@ -2328,14 +2515,17 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
     const PackedWeights& pk = w.pk;
     MARK();
     // per-call fills: run bounds of the s2 keys (k_runs writes those that
-    // occur), the list and chunk counters, the prediction-grid writers
-    // one-pass scan: the group-count bound of this call's cells (see ensure_workspace)
-    const int nv2 = E / (kCH * kSG) + 3, nv3 = E / (kCH * kSG3) + 3;
+    // occur), the list and group counters, the prediction-grid writers
+    // the group-count bound of this call's cells (see ensure_workspace), and
+    // whether a level's group list fits the key scan's LDS
+    const int nv = E / kGP + 3;
+    const bool gt2 = nk2 <= (uint32_t)kScanThreads && nv <= kGroupLds;
+    const bool gt3 = nk3 <= (uint32_t)kScanThreads && nv <= kGroupLds;
     FillSet f{};
     {
         int* arr[kFills] = {w.st2, w.en2, w.counts, w.last3, w.cnt3, w.ghist, w.ghist3};
         const int len[kFills] = {(int)nk2, (int)nk2, 16, have_head ? (int)nk3 : 0,
-                                 have_head ? (int)nk3 : 0, nv2, nv3};
+                                 have_head ? (int)nk3 : 0, gt2 ? 0 : nv, gt3 ? 0 : nv};
         const int val[kFills] = {0, 0, 0, -1, 0, 0, 0};
         for (int i = 0; i < kFills; ++i) {
             f.p[i] = arr[i];
@@ -2345,7 +2535,7 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
     }
     // ---- decode (and the fills); stable radix sort of the records by s2 key --
     {
-        const int ndec = (int)grid1(E, kDecRec), fblk = (int)grid1(std::max<int>(std::max<int>((int)nk2, 16), nv3), 256);
+        const int ndec = (int)grid1(E, kDecRec), fblk = (int)grid1(std::max<int>(std::max<int>((int)nk2, 16), nv), 256);
         const int npk = (int)((PackLayout<true>::off[8] + 255) / 256);
         hipLaunchKernelGGL(k_decode, dim3(ndec + fblk * kFills + npk + 1), dim3(256), 0, st, E, tab,
                            w.bd, G, w.X0, w.cell2, w.owner, w.ka, w.va, ndec, f, fblk, psrc,
@@ -2383,29 +2573,42 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
     uint32_t* const V2 = vin;
     uint32_t* const K3 = kout;
     uint32_t* const V3 = vout;
-    // ---- counters, tdrop_s2, the pass-2 list, s2 pair and chunk tables -----
+    // ---- counters, tdrop_s2, the pass-2 list, s2 pair and group tables -----
     if (passes == 1 && nk2 <= (uint32_t)kScanThreads) {
         // the one pass's histogram holds the run bounds: the key tables and
         // their scans in one workgroup
         const KeyHist kh{G.C2, G.W2, G.H2, T, G.window, (const int*)w.bh, w.st2, w.en2, w.bd,
                          w.old2};
-        hipLaunchKernelGGL(k_keyscan<true>, dim3(1), dim3(kScanThreads), 0, st, (int)nk2,
-                           (const int*)nullptr, w.pst2, w.pen2, w.coff2, w.counts + 2, w.n2,
-                           w.off2, w.counts + 0, kh);
+        if (gt2)
+            hipLaunchKernelGGL((k_keyscan<true, true>), dim3(1), dim3(kScanThreads), 0, st, (int)nk2,
+                               (const int*)nullptr, w.pst2, (int*)nullptr, w.goff2, w.n2, w.off2,
+                               w.counts + 0, kh, GroupTab{nv, w.glist, w.counts + 6});
+        else
+            hipLaunchKernelGGL((k_keyscan<true, false>), dim3(1), dim3(kScanThreads), 0, st, (int)nk2,
+                               (const int*)nullptr, w.pst2, (int*)nullptr, w.goff2, w.n2, w.off2,
+                               w.counts + 0, kh, GroupTab{});
     } else {
         hipLaunchKernelGGL(k_runs, dim3(grid1(E, 256)), dim3(256), 0, st, E, K2, nk2, w.st2, w.en2);
         hipLaunchKernelGGL(k_keys2, dim3(grid1(nk2, 256)), dim3(256), 0, st, nk2, G.C2, G.W2, G.H2,
-                           w.st2, w.en2, w.bd, G.window, w.old2, w.n2, w.pen2);
-        hipLaunchKernelGGL(k_keyscan<false>, dim3(1), dim3(kScanThreads), 0, st, (int)nk2, w.pen2,
-                           w.pst2, w.pen2, w.coff2, w.counts + 2, w.n2, w.off2, w.counts + 0,
-                           KeyHist{});
+                           w.st2, w.en2, w.bd, G.window, w.old2, w.n2, w.pcnt);
+        if (gt2)
+            hipLaunchKernelGGL((k_keyscan<false, true>), dim3(1), dim3(kScanThreads), 0, st, (int)nk2,
+                               w.pcnt, w.pst2, (int*)nullptr, w.goff2, w.n2, w.off2, w.counts + 0,
+                               KeyHist{}, GroupTab{nv, w.glist, w.counts + 6});
+        else
+            hipLaunchKernelGGL((k_keyscan<false, false>), dim3(1), dim3(kScanThreads), 0, st, (int)nk2,
+                               w.pcnt, w.pst2, (int*)nullptr, w.goff2, w.n2, w.off2, w.counts + 0,
+                               KeyHist{}, GroupTab{});
     }
     {
         const unsigned nbr = grid1(E, 256);
-        hipLaunchKernelGGL(k_s2_tables, dim3(nbr + grid1(nk2, 4)), dim3(256), 0, st, E, (int)nbr,
-                           K2, V2, nk2, G.C2, G.W2, G.H2, w.st2, w.en2, w.pst2, w.pen2, w.coff2,
-                           w.old2, w.off2, G.window, w.pass2, w.list2, w.pos2, w.pneed2, w.ckey2,
-                           w.cbeg2, w.cend2, w.ghist, w.gw);
+        hipLaunchKernelGGL(k_s2_tables, dim3(nbr + (gt2 ? 0u : grid1(nk2, 256))), dim3(256), 0, st, E,
+                           (int)nbr, K2, V2, nk2, G.C2, G.W2, G.H2, w.st2, w.en2, w.pst2, w.old2,
+                           w.off2, G.window, w.pass2, w.list2, w.pent2, w.gcnt, w.gend, w.ghist, w.gw);
+        if (!gt2)
+            hipLaunchKernelGGL(k_group_order, dim3(1), dim3(kScanThreads), 0, st, (int)nk2, nv, w.pst2,
+                               w.goff2, w.gcnt, w.gend, w.ghist, w.gw, w.gstart, w.gbase, w.glist,
+                               w.counts + 6);
     }
     // The s3 ordering needs only the s2 order, pass2 and the old counters, so
     // it runs on the side stream while L4 and L5 run here; L6 waits for it.
@@ -2426,61 +2629,52 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
     const long long Pw = G.window <= 1 ? 256 : (256 + G.window - 1) / G.window;
     const int nmax2 = (int)std::min<long long>(E, ((long long)E * Pw + 255) / 256 + 2LL * nk2);
     const int nmax3 = (int)std::min<long long>(nmax2, ((long long)nmax2 * Pw + 255) / 256 + 2LL * nk3);
-    const unsigned tiles2 = grid1(nmax2, kTM), tiles3 = grid1(nmax3, kTM);
-    // persistent projection grids (80-record tiles loop over the workgroups):
-    // measured at 200k records (2500 tiles), L4 is fastest with 6 workgroups
-    // per CU, L5 with 5 (both: all resident, about two tiles each); 64-record
-    // tiles (3125, some workgroups running a third) were 10% slower.
-    const unsigned tilesP = grid1(E, kTMP);
-    const unsigned cus = w.cus > 0 ? (unsigned)w.cus : tilesP;
-    const unsigned gridP4 = std::min(tilesP, 6u * cus);
-    const unsigned gridP5 = std::min(tilesP, 5u * cus);
-    const unsigned char* all = nullptr;             // every pair's record needs h
-    // L4's and L5's h, compact (pairs, 48), behind their (pairs, 96) rows
-    float* const Hc = w.QVG + (size_t)w.cap * kPatch * 2 * SSLA_C2;
-    // S: the recurrence of layer LI over the chunk tables of level LV (2: s2,
-    // 3: s3; n_chunks in counts[NC]), h written at HOUT (rows of HS floats)
-    // where the pair's record needs the output (NEED, or every pair), in one
-    // pass (k_scan; ticket counter counts[8 + LI], group count counts[NG]).
+    const unsigned tiles3 = grid1(nmax3, kTM);
+    const int* const no_count = nullptr;
+    const int* const no_list = nullptr;
+    // P + S of layer LI over the groups of level LV (their count in
+    // counts[NG], ticket counter counts[8 + LI]): h rows to HR where the pair's
+    // record needs the output (ALL: every pair's).  Two workgroups of k_pscan
+    // fit a CU (LDS), and the grid is what is resident at once, or the groups
+    // the call can have: full groups, a tail per cell of more than kGW pairs
+    // and the shared ones, one per window of kGW.
     const unsigned long long wait_ticks = (unsigned long long)std::max(w.clk_khz, 1) * 500ull;
-#define SCAN1(OUT, HS, SGV, LI, LV, NG, GL, NEED, HOUT, CELLS, GRID)                                  \
+    const unsigned cus = w.cus > 0 ? (unsigned)w.cus : 256u;
+    auto group_bound = [](long long recs, long long nk) {
+        const long long p = recs * kPatch, small = p / kGW + 1;
+        return p / kGP + 2 * std::min(nk, small);
+    };
+    auto ps_grid = [&](long long groups, int slabs) {
+        return (unsigned)std::min<long long>(groups * slabs, cus);
+    };
+    const unsigned gridS4 = ps_grid(group_bound(E, nk2), 1);
+    const unsigned gridS6 = ps_grid(group_bound(nmax2, nk3), SSLA_C3 / kPSC);
+#define PSCAN(IN, OUT, NT, LI, LV, NG, GL, ALL, XIN, CELLS, GRID)                                    \
     do {                                                                                            \
         unsigned tag_ = ++g_scan_tag;                                                               \
         if (tag_ == 0) tag_ = ++g_scan_tag;                                                         \
+        hipLaunchKernelGGL((k_pscan<IN, OUT, ALL, NT>), dim3(GRID), dim3(kPSThreads), 0, st,             \
+                           (const int*)(w.counts + NG), w.counts + 8 + LI, tag_, GL, w.pent##LV,     \
+                           XIN, pk.pp[LI], CELLS, w.bd, LI, w.HR, w.sw, w.scan_err, wait_ticks);    \
         MARK();                                                                                     \
         MARK();                                                                                     \
-        hipLaunchKernelGGL((k_scan<OUT, HS, SGV>), dim3(GRID), dim3(SGV * ((OUT + 63) / 64) * 64), 0, \
-                           st, (const int*)(w.counts + NG), w.counts + 8 + LI, tag_, GL,             \
-                           w.cbeg##LV, w.cend##LV, w.coff##LV, w.pst##LV, w.pen##LV, CELLS, w.bd,   \
-                           LI, NEED, w.QVG, HOUT, w.sw, w.scan_err, wait_ticks);                    \
+        MARK();                                                                                     \
         MARK();                                                                                     \
     } while (0)
-    // workgroups of the one-pass scans: one per group (at most one per kSG
-    // chunks plus one per key); those past the group count exit at once
-    const unsigned groups2 = (unsigned)(((size_t)E * kPatch / kCH + nk2 + 1) / kSG + nk2 + 1);
-    const unsigned groups3 = (unsigned)(((size_t)nmax2 * kPatch / kCH + nk3 + 1) / kSG3 + nk3 + 1);
     // ---- L4: 24 -> 48, all records ----------------------------------------
-    hipLaunchKernelGGL((k_qvg<SSLA_C1, SSLA_C2, true, kTMP>), dim3(gridP4), dim3(256), 0, st, E,
-                       (const int*)nullptr, (const int*)nullptr, w.X0, w.pos2, pk.pp[0], w.QVG, w.trash);
-    // [side] the s2 one-pass scan's ticket order, beside L4's projection
-    hipLaunchKernelGGL(k_group_order, dim3(1), dim3(kScanThreads), 0, s3, (int)nk2, nv2, kSG, w.pst2,
-                       w.pen2, w.ghist, w.gw, w.gstart, w.gbase, w.glist, w.counts + 6);
-    HIPCHK(hipEventRecord(w.s2_groups, s3));
-    MARK();
-    HIPCHK(hipStreamWaitEvent(st, w.s2_groups, 0));
-    SCAN1(SSLA_C2, SSLA_C2, kSG, 0, 2, 6, w.glist, all, Hc, G.C2, groups2);
-    hipLaunchKernelGGL((k_outt<SSLA_C1, SSLA_C2, 2, 1, 3, SSLA_C2>), dim3(grid1(E, 32)), dim3(64), 0,
-                       st, E, (const int*)nullptr, (const int*)nullptr, w.X0, w.pos2, Hc, pk.po[0],
+    PSCAN(SSLA_C1, SSLA_C2, true, 0, 2, 6, w.glist, true, w.X0, G.C2, gridS4);
+    hipLaunchKernelGGL((k_outt<SSLA_C1, SSLA_C2, 2, 1, 3>), dim3(grid1(E, 32)), dim3(64), 0, st, E,
+                       no_count, no_list, w.X0, w.cell2, 0, G.W2, G.W2, G.H2, w.HR, pk.po[0],
                        L[0].ln_gamma, L[0].ln_beta, w.X1);
     MARK();
-    // ---- [side] the s3 record order, tdrop_s3, s3 pair and chunk tables ---
+    // ---- [side] the s3 record order, tdrop_s3, s3 pair and group tables ---
     // (enqueued after L4's launches: the host needs a few microseconds per
     // launch, and L4 keeps the device busy meanwhile)
     hipLaunchKernelGGL(k_keys3a, dim3(grid1(nk3, 256)), dim3(256), 0, s3, nk3, G, w.n2, w.bd,
                        w.t3, w.n3);
-    hipLaunchKernelGGL(k_keyscan<false>, dim3(1), dim3(kScanThreads), 0, s3, (int)nk3, w.t3, w.st3,
-                       w.en3, (int*)nullptr, (int*)nullptr, w.n3, w.off3, w.counts + 1,
-                       KeyHist{});
+    hipLaunchKernelGGL((k_keyscan<false, false>), dim3(1), dim3(kScanThreads), 0, s3, (int)nk3, w.t3,
+                       w.st3, w.en3, (int*)nullptr, w.n3, w.off3, w.counts + 1, KeyHist{},
+                       GroupTab{});
     hipLaunchKernelGGL(k_place3, dim3(grid1(nmax2, 256)), dim3(256), 0, s3, (const int*)(w.counts + 0),
                        w.list2, w.bd, G, w.cell2, w.sidx, V2, w.st2, w.en2, w.old2, w.st3, K3, V3,
                        w.key3g);
@@ -2488,49 +2682,47 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
                        K3, V3, nk3, G.C3, w.st3, w.off3, w.bd, G.window, w.owner,
                        have_head ? 1 : 0, w.pass3, w.list3, w.last3, w.cnt3);
     hipLaunchKernelGGL(k_keys3b, dim3(grid1(nk3, 256)), dim3(256), 0, s3, nk3, G, w.t3, w.bd,
-                       w.pen3);
-    hipLaunchKernelGGL(k_keyscan<false>, dim3(1), dim3(kScanThreads), 0, s3, (int)nk3, w.pen3, w.pst3,
-                       w.pen3, w.coff3, w.counts + 3, (const int*)nullptr, (int*)nullptr,
-                       (int*)nullptr, KeyHist{});
-    hipLaunchKernelGGL(k_chunks, dim3(grid1(nk3, 4)), dim3(256), 0, s3, nk3, w.pst3, w.pen3,
-                       w.coff3, w.ckey3, w.cbeg3, w.cend3, w.ghist3, w.gw3);
-    hipLaunchKernelGGL(k_group_order, dim3(1), dim3(kScanThreads), 0, s3, (int)nk3, nv3, kSG3, w.pst3,
-                       w.pen3, w.ghist3, w.gw3, w.gstart3, w.gbase3, w.glist3, w.counts + 7);
+                       w.pcnt);
+    if (gt3) {
+        hipLaunchKernelGGL((k_keyscan<false, true>), dim3(1), dim3(kScanThreads), 0, s3, (int)nk3,
+                           w.pcnt, w.pst3, (int*)nullptr, w.goff3, (const int*)nullptr, (int*)nullptr,
+                           (int*)nullptr, KeyHist{}, GroupTab{nv, w.glist3, w.counts + 7});
+    } else {
+        hipLaunchKernelGGL((k_keyscan<false, false>), dim3(1), dim3(kScanThreads), 0, s3, (int)nk3,
+                           w.pcnt, w.pst3, (int*)nullptr, w.goff3, (const int*)nullptr, (int*)nullptr,
+                           (int*)nullptr, KeyHist{}, GroupTab{});
+        hipLaunchKernelGGL(k_key_groups, dim3(grid1(nk3, 256)), dim3(256), 0, s3, nk3, w.pst3, w.gcnt3,
+                           w.gend3, w.ghist3, w.gw3);
+        hipLaunchKernelGGL(k_group_order, dim3(1), dim3(kScanThreads), 0, s3, (int)nk3, nv, w.pst3,
+                           w.goff3, w.gcnt3, w.gend3, w.ghist3, w.gw3, w.gstart3, w.gbase3, w.glist3,
+                           w.counts + 7);
+    }
     hipLaunchKernelGGL(k_pair_rank, dim3(grid1(nmax2, 256)), dim3(256), 0, s3, E,
                        (const int*)(w.counts + 0), K3, V3, nk3, G.C3, G.W3, G.H3, w.st3, w.en3,
-                       w.pst3, w.pos3, w.pneed3, w.pass3);
+                       w.pst3, w.pent3, w.pass3);
     HIPCHK(hipEventRecord(w.s3_ordered, s3));
     HIPCHK(hipGetLastError());
     // ---- L5: 48 -> 48, state for all records, output for pass2 ---------------
-    hipLaunchKernelGGL((k_qvg<SSLA_C2, SSLA_C2, true, kTMP>), dim3(gridP5), dim3(256), 0, st, E,
-                       (const int*)nullptr, (const int*)nullptr, w.X1, w.pos2, pk.pp[1], w.QVG, w.trash);
-    MARK();
-    SCAN1(SSLA_C2, SSLA_C2, kSG, 1, 2, 6, w.glist, w.pneed2, Hc, G.C2, groups2);
-    hipLaunchKernelGGL((k_outt<SSLA_C2, SSLA_C2, kOutRT5, kOutKS5, 1, SSLA_C2>), dim3(grid1(nmax2, 16 * kOutRT5)),
-                       dim3(64 * kOutKS5), 0,
-                       st, E, (const int*)(w.counts + 0), w.list2, w.X1, w.pos2, Hc, pk.po[1],
-                       L[1].ln_gamma, L[1].ln_beta, w.X2);
+    PSCAN(SSLA_C2, SSLA_C2, true, 1, 2, 6, w.glist, false, w.X1, G.C2, gridS4);
+    hipLaunchKernelGGL((k_outt<SSLA_C2, SSLA_C2, kOutRT5, kOutKS5>), dim3(grid1(nmax2, 16 * kOutRT5)),
+                       dim3(64 * kOutKS5), 0, st, E, (const int*)(w.counts + 0), w.list2, w.X1,
+                       w.cell2, 0, G.W2, G.W2, G.H2, w.HR, pk.po[1], L[1].ln_gamma, L[1].ln_beta,
+                       w.X2);
     MARK();
     // ---- L6: 48 -> 96, pass2 records ------------------------------------------
     HIPCHK(hipStreamWaitEvent(st, w.s3_ordered, 0));
-    hipLaunchKernelGGL((k_qvg<SSLA_C2, SSLA_C3, false, kTM, 2>), dim3(tiles2 * 2), dim3(256), 0, st, E,
-                       (const int*)(w.counts + 0), w.list2, w.X2, w.pos3, pk.pp[2], w.QVG, w.trash);
-    MARK();
-    SCAN1(SSLA_C3, 2 * SSLA_C3, kSG3, 2, 3, 7, w.glist3, all, w.QVG, G.C3, groups3);
+    PSCAN(SSLA_C2, SSLA_C3, false, 2, 3, 7, w.glist3, true, w.X2, G.C3, gridS6);
     hipLaunchKernelGGL((k_outt<SSLA_C2, SSLA_C3, kOutRT6, kOutKS6>), dim3(grid1(nmax2, 16 * kOutRT6)),
-                       dim3(64 * kOutKS6), 0, st, E,
-                       (const int*)(w.counts + 0), w.list2, w.X2, w.pos3, w.QVG, pk.po[2],
-                       L[2].ln_gamma, L[2].ln_beta, w.X3);
+                       dim3(64 * kOutKS6), 0, st, E, (const int*)(w.counts + 0), w.list2, w.X2,
+                       w.cell2, 1, G.W2, G.W3, G.H3, w.HR, pk.po[2], L[2].ln_gamma, L[2].ln_beta,
+                       w.X3);
     MARK();
     // ---- L7: 96 -> 96, state for pass2, output for pass3 ----------------------
-    hipLaunchKernelGGL((k_qvg<SSLA_C3, SSLA_C3, false, kTM, 4>), dim3(tiles2 * 4), dim3(256), 0, st, E,
-                       (const int*)(w.counts + 0), w.list2, w.X3, w.pos3, pk.pp[3], w.QVG, w.trash);
-    MARK();
-    SCAN1(SSLA_C3, 2 * SSLA_C3, kSG3, 3, 3, 7, w.glist3, w.pneed3, w.QVG, G.C3, groups3);
+    PSCAN(SSLA_C3, SSLA_C3, false, 3, 3, 7, w.glist3, false, w.X3, G.C3, gridS6);
     hipLaunchKernelGGL((k_outt<SSLA_C3, SSLA_C3, kOutRT7, kOutKS7>), dim3(grid1(nmax3, 16 * kOutRT7)),
-                       dim3(64 * kOutKS7), 0, st, E,
-                       (const int*)(w.counts + 1), w.list3, w.X3, w.pos3, w.QVG, pk.po[3],
-                       L[3].ln_gamma, L[3].ln_beta, w.X4);
+                       dim3(64 * kOutKS7), 0, st, E, (const int*)(w.counts + 1), w.list3, w.X3,
+                       w.cell2, 1, G.W2, G.W3, G.H3, w.HR, pk.po[3], L[3].ln_gamma, L[3].ln_beta,
+                       w.X4);
     MARK();
     HIPCHK(hipGetLastError());
     // ---- head ------------------------------------------------------------------
@@ -2552,7 +2744,7 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
     HIPCHK(hipGetLastError());
     MARK();
 #undef MARK
-#undef SCAN1
+#undef PSCAN
     end.finish();
     if (phase_ms) {
         // this call's events join the pending ones (read below when sync is
@@ -2573,7 +2765,7 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
     if (sync) {
         HIPCHK(hipStreamSynchronize(st));
         if (__atomic_exchange_n(w.scan_err, 0, __ATOMIC_RELAXED)) {
-            set_error("drain: a wait of the one-pass scan ran out (results are invalid)");
+            set_error("drain: a wait of the recurrence's look-back ran out (results are invalid)");
             return SSLA_ERR_HIP;
         }
         // every earlier call finished before this one's kernels started

@@ -115,6 +115,39 @@ struct OutPackT {
     static_assert(OUT % kMT == 0 && IN % 4 == 0 && (IP || IN == OUT), "tile shapes");
 };
 
+// The v and g projections of the whole-ring drain (k_pscan): A-operand copies
+// of qvgIn's v and g columns with OutPackT's K order, so a lane's B values are
+// float4 pieces of a record's input row.  Items are ordered as a workgroup
+// runs them, per delta and slab of 48 channels: the slab's three v tiles, then
+// its three g tiles.
+//   items (delta, slab, j), groups t < KG, lane, i < 4:
+//     qvgIn[delta][kidx(t, g, i)][(j < 3 ? OUT : 2 OUT) + 48 slab + 16 (j % 3) + lane % 16]
+template <int IN, int OUT>
+struct ProjPackT {
+    using O = OutPackT<IN, OUT>;
+    static constexpr int KG = O::KG, NS = OUT / 48;
+    static __host__ __device__ constexpr int steps(int t) { return O::steps(t); }
+    static __host__ __device__ constexpr int kidx(int t, int g, int i) { return O::kidx(t, g, i); }
+    static constexpr size_t PACKED = (size_t)9 * NS * 6 * KG * 256;   // floats
+    static_assert(OUT % 48 == 0, "slabs");
+};
+
+// element q of a layer's ProjPackT region
+template <int IN, int OUT>
+__device__ __forceinline__ float projt_elem(const float* __restrict__ qvgIn, size_t q) {
+    using P = ProjPackT<IN, OUT>;
+    const int i = (int)(q & 3), lane = (int)((q >> 2) & 63), g = lane >> 4;
+    size_t r = q >> 8;
+    const int t = (int)(r % P::KG);
+    r /= P::KG;
+    const int j = (int)(r % 6);
+    r /= 6;
+    const int slab = (int)(r % P::NS), d = (int)(r / P::NS);
+    const int k = P::kidx(t, g, i);
+    const int c = (j < 3 ? OUT : 2 * OUT) + 48 * slab + 16 * (j % 3) + (lane & 15);
+    return i < P::steps(t) && k < IN ? qvgIn[((size_t)d * IN + k) * (3 * OUT) + c] : 0.f;
+}
+
 // element q of a layer's OutPackT region
 template <int IN, int OUT>
 __device__ __forceinline__ float outt_elem(const float* __restrict__ qvgIn,
@@ -192,13 +225,13 @@ struct PackSrc {
 // Floats of one layer's projection copy and contraction copy.
 template <int IN, int OUT, bool D>
 struct LayerPack {
-    static constexpr size_t NP = ProjPack<IN, OUT>::PACKED;
+    static constexpr size_t NP = D ? ProjPackT<IN, OUT>::PACKED : ProjPack<IN, OUT>::PACKED;
     static constexpr size_t NO = D ? OutPackT<IN, OUT>::PACKED : OutPack<IN, OUT>::PACKED;
 };
 
 // Buffer order: L4 projection, L4 contraction, L5 ..., L7 contraction.
-// D selects the transposed contraction of the whole-ring drain (OutPackT)
-// instead of the K split of the batch kernels.
+// D selects the whole-ring drain's copies (ProjPackT, the transposed
+// contraction OutPackT) instead of the batch kernels' (ProjPack, the K split).
 template <bool D>
 struct PackLayout {
     using A = LayerPack<SSLA_C1, SSLA_C2, D>;
@@ -216,6 +249,12 @@ struct PackLayout {
 };
 
 template <int IN, int OUT, bool D>
+__device__ __forceinline__ float proj_any(const float* qvgIn, size_t q) {
+    if constexpr (D) return projt_elem<IN, OUT>(qvgIn, q);
+    else return proj_elem<IN, OUT>(qvgIn, q);
+}
+
+template <int IN, int OUT, bool D>
 __device__ __forceinline__ float out_any(const float* qvgIn, const float* goW, const float* ip,
                                          size_t q) {
     if constexpr (D) return outt_elem<IN, OUT>(qvgIn, goW, ip, q);
@@ -227,13 +266,13 @@ template <bool D>
 __device__ __forceinline__ void pack_elem(const PackSrc& s, float* __restrict__ buf, size_t q) {
     using L = PackLayout<D>;
     float v;
-    if (q < L::off[1]) v = proj_elem<SSLA_C1, SSLA_C2>(s.qvgIn[0], q);
+    if (q < L::off[1]) v = proj_any<SSLA_C1, SSLA_C2, D>(s.qvgIn[0], q);
     else if (q < L::off[2]) v = out_any<SSLA_C1, SSLA_C2, D>(s.qvgIn[0], s.goW[0], s.ip[0], q - L::off[1]);
-    else if (q < L::off[3]) v = proj_elem<SSLA_C2, SSLA_C2>(s.qvgIn[1], q - L::off[2]);
+    else if (q < L::off[3]) v = proj_any<SSLA_C2, SSLA_C2, D>(s.qvgIn[1], q - L::off[2]);
     else if (q < L::off[4]) v = out_any<SSLA_C2, SSLA_C2, D>(s.qvgIn[1], s.goW[1], s.ip[1], q - L::off[3]);
-    else if (q < L::off[5]) v = proj_elem<SSLA_C2, SSLA_C3>(s.qvgIn[2], q - L::off[4]);
+    else if (q < L::off[5]) v = proj_any<SSLA_C2, SSLA_C3, D>(s.qvgIn[2], q - L::off[4]);
     else if (q < L::off[6]) v = out_any<SSLA_C2, SSLA_C3, D>(s.qvgIn[2], s.goW[2], s.ip[2], q - L::off[5]);
-    else if (q < L::off[7]) v = proj_elem<SSLA_C3, SSLA_C3>(s.qvgIn[3], q - L::off[6]);
+    else if (q < L::off[7]) v = proj_any<SSLA_C3, SSLA_C3, D>(s.qvgIn[3], q - L::off[6]);
     else v = out_any<SSLA_C3, SSLA_C3, D>(s.qvgIn[3], s.goW[3], s.ip[3], q - L::off[7]);
     buf[q] = v;
 }
