@@ -322,7 +322,7 @@ def launch_work(flops, byts, iface):
 
 
 # kernel of each timed launch of the whole-ring drain (ssla-rt_amd/csrc/drain_scan.hip)
-PHASE_KERNEL = {"order": "ordering kernels", "head": "k_head + k_pred_*", "emit": "k_emit"}
+PHASE_KERNEL = {"order": "ordering kernels", "head": "k_head", "emit": "k_emit"}
 for _L, (_i, _o) in zip(("L4", "L5", "L6", "L7"), ((C1, C2), (C2, C2), (C2, C3), (C3, C3))):
     # projection and recurrence are one launch, in the proj slot
     PHASE_KERNEL[f"{_L}.proj"] = f"k_pscan<{_i}, {_o}>"
@@ -465,7 +465,7 @@ def halo_divergence(stub_dir, rec, n, p2o, p3o, feat_o, H2, W2, blocks=8):
 
 def _roofline_phase(per):
     """The phase of the longest single-kernel launch (the ordering phase is
-    several kernels, the head two)."""
+    several kernels; the head's work is counted for owned records only)."""
     single = {k: v for k, v in per.items() if k not in ("order", "head")}
     return max(single, key=single.get)
 
@@ -624,21 +624,22 @@ TRAFFIC_PHASES = {
     "k_pscan<96, 96>": ["L7.proj"],
     "k_outt<24, 48, 2, 1>": ["L4.out"], "k_outt<48, 48, 1, 3>": ["L5.out"],
     "k_outt<48, 96, 1, 3>": ["L6.out"], "k_outt<96, 96, 1, 3>": ["L7.out"],
-    "k_head": ["head"], "k_head_linear": ["head"], "k_pred_write": ["head"], "k_emit": ["emit"],
+    "k_head": ["head"], "k_head_linear": ["head"], "k_emit": ["emit"],
 }
-ORDER_KERNELS = ("k_decode", "k_rs_hist", "k_exscan", "k_rs_scatter", "k_runs", "k_keys2",
+ORDER_KERNELS = ("k_decode", "k_small_order", "k_rs_hist", "k_exscan", "k_rs_scatter", "k_runs", "k_keys2",
                  "k_keyscan", "k_s2_tables", "k_pair_rank", "k_key_groups", "k_keys3a", "k_place3",
                  "k_tdrop3", "k_keys3b", "k_group_order")
 
 
 def _traffic_key(k: str):
     """The TRAFFIC_PHASES key of kernel name k: the key itself, or a key
+    without template arguments that names k's kernel, or one
     whose template arguments are the first arguments of k's (the launch
     parameters that follow them -- tile sizes, waves per SIMD, row strides --
     do not change the phase)."""
     for key in TRAFFIC_PHASES:
         base = key[:-1]
-        if k == key or (key.endswith(">") and k.startswith(base) and k[len(base)] in ",>"):
+        if k == key or k.split("<")[0] == key or (key.endswith(">") and k.startswith(base) and k[len(base)] in ",>"):
             return key
     return None
 
@@ -710,8 +711,6 @@ def trace_summary(trace_dir, command):
             continue
         ph = TRAFFIC_PHASES[key]
         lab = ph[seen[key] % len(ph)]
-        if lab == "head":                         # two kernels: kept apart
-            lab += ":" + k.split("<")[0]
         seen[key] += 1
         tot[lab] += (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) * 1e-6
         cnt[lab] += 1

@@ -149,7 +149,7 @@ int ssla_hip_drain_n2(const HybridS2S3Config* cfg,
 
 #define SSLA_DRAIN_PHASES 23
 /* Phase order of SslaHipDrainOpts.phase_ms (one kernel launch each, except
- * 0, 21): 0 ordering (decode, sorts, tdrop decisions, pair and group
+ * 0): 0 ordering (decode, sorts, tdrop decisions, pair and group
  * tables); per layer the projection of v, g with the recurrence over them in
  * the first of four slots (the other three are empty), then the contraction
  * (q, q*h, goW, residual, LayerNorm): L4 1-5, L5 6-10, L6 11-15, L7 16-20;

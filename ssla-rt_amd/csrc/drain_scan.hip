@@ -588,6 +588,22 @@ struct GroupTab {
     int* n_groups;
 };
 
+// The group list of at most kScanThreads keys (one per thread of the
+// workgroup) from pair starts pst (nk + 1) and word slots go; hist and start
+// hold gt.nv entries, hist zero before.  All arrays in LDS.
+__device__ __forceinline__ void group_list_lds(int nk, const int* pst, const int* go, int* hist,
+                                               int* start, int* lds, GroupTab gt) {
+    const int k = (int)threadIdx.x;
+    int gc = 0, pend = 0, place = 0;
+    if (k < nk) gc = key_groups(k, nk, pst, &pend);
+    if (gc > 0) place = atomicAdd(&hist[gc], 1);
+    __syncthreads();
+    // (the base table takes hist's place: hist is read before it is written)
+    group_order(nk, gt.nv, hist, start, hist, lds, [&](int q) {
+        return LeadKey{gc, pend, place, pst[q], go[q], pend > pst[q + 1] ? kGMulti : 0};
+    }, gt.glist, gt.n_groups);
+}
+
 template <bool KH, bool GT>
 __global__ void __launch_bounds__(kScanThreads)
 k_keyscan(int nk, const int* cnt, int* __restrict__ start, int* end, int* __restrict__ goff,
@@ -676,15 +692,7 @@ k_keyscan(int nk, const int* cnt, int* __restrict__ start, int* end, int* __rest
     if constexpr (GT) {
         if (threadIdx.x == 0) spst[nk] = carry;
         __syncthreads();
-        const int k = (int)threadIdx.x;
-        int gc = 0, pend = 0, place = 0;
-        if (k < nk) gc = key_groups(k, nk, spst, &pend);
-        if (gc > 0) place = atomicAdd(&shist[gc], 1);
-        __syncthreads();
-        // (the base table takes hist's place: hist is read before it is written)
-        group_order(nk, gt.nv, shist, sstart, shist, lds, [&](int q) {
-            return LeadKey{gc, pend, place, spst[q], sgo[q], pend > spst[q + 1] ? kGMulti : 0};
-        }, gt.glist, gt.n_groups);
+        group_list_lds(nk, spst, sgo, shist, sstart, lds, gt);
     }
 }
 
@@ -953,9 +961,11 @@ rank_segment(uint32_t ks, int l0, int l1, bool in, uint32_t g, const uint32_t* _
 }
 
 // A wave's lanes are consecutive records of the sorted order.  When they
-// span at most kSegMax keys (the usual case), each key's segment is ranked
-// by rank_segment; otherwise each lane searches the 24 whole runs, all 24
+// span at most kSegMax keys (the usual case of a large call), each key's segment
+// is ranked by rank_segment; otherwise, and always when vals is in LDS (LV: a
+// small call, whose runs are short), each lane searches the 24 whole runs, all 24
 // binary searches advanced together.
+template <bool LV>
 __device__ __forceinline__ void
 pair_rank_at(int i, int n, const uint32_t* __restrict__ keys,
              const uint32_t* __restrict__ vals, uint32_t nk, int C, int W, int H,
@@ -974,7 +984,7 @@ pair_rank_at(int i, int n, const uint32_t* __restrict__ keys,
     int r25[25];
     #pragma unroll
     for (int c = 0; c < 25; ++c) r25[c] = 0;
-    if (nseg <= kSegMax) {
+    if (!LV && nseg <= kSegMax) {
         unsigned long long left = kmask;
         while (left) {
             const int l0 = (int)__ffsll((long long)left) - 1;
@@ -1036,19 +1046,38 @@ pair_rank_at(int i, int n, const uint32_t* __restrict__ keys,
     }
 }
 
+// A small call's sorted records in LDS: the searches of a wave are dependent
+// loads, and a small call has too few waves to hide them (at 4100 records the s2
+// tables took 47 us with the searches in memory).
+constexpr int kSmallRec = 8 * kScanThreads;
+
+__device__ __forceinline__ void stage_vals(int n, const uint32_t* __restrict__ vals, uint32_t* sv) {
+    for (int i = threadIdx.x; i < n; i += blockDim.x) sv[i] = vals[i];
+    __syncthreads();
+}
+
+template <bool SMALL>
 __global__ void __launch_bounds__(256)
 k_pair_rank(int n_max, const int* __restrict__ n_dev, const uint32_t* __restrict__ keys,
             const uint32_t* __restrict__ vals, uint32_t nk, int C, int W, int H,
             const int* __restrict__ st, const int* __restrict__ en, const int* __restrict__ pst,
             uint2* __restrict__ pent, const unsigned char* __restrict__ pass) {
-    pair_rank_at(blockIdx.x * blockDim.x + threadIdx.x, n_dev ? *n_dev : n_max, keys, vals, nk,
-                 C, W, H, st, en, pst, pent, pass, false);
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, n = n_dev ? *n_dev : n_max;
+    if constexpr (SMALL) {
+        __shared__ uint32_t sv[kSmallRec];
+        if ((int)(blockIdx.x * blockDim.x) >= n) return;
+        stage_vals(n, vals, sv);
+        pair_rank_at<true>(i, n, keys, sv, nk, C, W, H, st, en, pst, pent, pass, false);
+    } else {
+        pair_rank_at<false>(i, n, keys, vals, nk, C, W, H, st, en, pst, pent, pass, false);
+    }
 }
 
 // The s2 level's tables that need only the sorted order and the key scan, in
 // one launch: per sorted record (blocks [0, nbr)) its tdrop_s2 decision and
 // list slot (tdrop2_at) and its pair ranks; per key (blocks nbr.., when the key
 // scan did not build the group list) the groups it leads.
+template <bool SMALL>
 __global__ void __launch_bounds__(256)
 k_s2_tables(int n, int nbr, const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,
             uint32_t nk, int C, int W, int H, const int* __restrict__ st,
@@ -1064,7 +1093,318 @@ k_s2_tables(int n, int nbr, const uint32_t* __restrict__ keys, const uint32_t* _
     }
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const bool take = tdrop2_at(i, n, keys, vals, nk, st, old, off, window, pass, list);
-    pair_rank_at(i, n, keys, vals, nk, C, W, H, st, en, pst, pent, nullptr, take);
+    if constexpr (SMALL) {
+        __shared__ uint32_t sv[kSmallRec];
+        stage_vals(n, vals, sv);
+        pair_rank_at<true>(i, n, keys, sv, nk, C, W, H, st, en, pst, pent, nullptr, take);
+    } else {
+        pair_rank_at<false>(i, n, keys, vals, nk, C, W, H, st, en, pst, pent, nullptr, take);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The ordering of a small call (k_small_order): workgroup 0 does, in LDS, what
+// k_decode's keys, the radix sort and the key scan do in five launches for
+// larger calls (ALL: the pair tables and the whole s3 ordering too, thirteen
+// launches); the other workgroups copy the input rows, rebuild the weight copies
+// and write the block table.  A small call's launches are latency, not work,
+// but one workgroup's work grows with the records: ALL takes 40 us at 300
+// records, where the launches it replaces took 110 on the call's critical path,
+// and would take 220 at 4100 (the pair ranks 113 of them), so it stops at one
+// record per thread; the sort and key tables alone take 27 us at 4100 records
+// against about 70, and stop at what the LDS holds (kSmallRec).
+// ---------------------------------------------------------------------------
+constexpr int kSmallAll = kScanThreads;          // records of an ALL call
+constexpr int kSmallGroups = kSmallRec / kGP + 3;
+constexpr int kSmallWaves = kScanThreads / 64;
+
+struct SmallOut {
+    int* cell2;
+    unsigned char *owner, *pass2, *pass3;
+    int *list2, *list3, *counts, *last3, *cnt3;
+    uint32_t* key3g;
+    uint2 *pent2, *pent3;
+    int4 *glist2, *glist3;
+    int have_head;
+    // not ALL: the tables of the launches that follow
+    uint32_t *keys2, *vals2;
+    int *sidx, *st2, *en2, *pst2, *n2, *off2;
+    unsigned char* old2;
+};
+
+struct SmallLds {
+    uint32_t v2[kSmallRec], k2[kSmallRec];       // records in s2 order, their keys
+    unsigned short key[kSmallRec];               // by record: s2 key | owner << 15
+    union {
+        unsigned short wc[kSmallWaves][kScanThreads + 2];    // sort: counts per wave and key
+        struct {
+            uint32_t v3[kSmallAll], k3[kSmallAll];           // pass-2 records in s3 order
+        };
+    };
+    int st[kScanThreads + 1], pst[kScanThreads + 1], cur[kScanThreads + 1], go[kScanThreads];
+    int n2[kScanThreads], off[kScanThreads];
+    unsigned char old[kScanThreads];
+    int hist[kSmallGroups], start[kSmallGroups];
+    int last[kScanThreads / 4], cnt[kScanThreads / 4];
+    int lds[2 * (kScanThreads / 64)];
+};
+static_assert(sizeof(SmallLds) <= 160 * 1024 - 256, "LDS of the small ordering");
+
+// exclusive scan over the workgroup, one value per thread (k < n): out[k], and
+// out[n] = the sum
+__device__ __forceinline__ int scan_keys(int v, int n, int* out, int* lds) {
+    int total;
+    const int k = (int)threadIdx.x, x = block_exscan(k < n ? v : 0, lds, &total);
+    if (k < n) out[k] = x;
+    if (k == 0) out[n] = total;
+    return total;
+}
+
+// pairs of key k: the run lengths (st) of its 3 x 3 neighbourhood
+__device__ __forceinline__ int pair_count(int k, int C, int W, int H, const int* st) {
+    const int b = k / C, cell = k % C, ty = cell / W, tx = cell % W;
+    int np = 0;
+    #pragma unroll
+    for (int oy = -1; oy <= 1; ++oy)
+        #pragma unroll
+        for (int ox = -1; ox <= 1; ++ox) {
+            const int sy = ty + oy, sx = tx + ox;
+            if (sy < 0 || sy >= H || sx < 0 || sx >= W) continue;
+            const int s = b * C + sy * W + sx;
+            np += st[s + 1] - st[s];
+        }
+    return np;
+}
+
+template <bool ALL>
+__global__ void __launch_bounds__(kScanThreads)
+k_small_order(int E, BlockTable tab, BlockDesc* __restrict__ bd_out, Geometry G,
+              float* __restrict__ X0, SmallOut o, PackSrc ps, float* __restrict__ pbuf, int npk) {
+    __shared__ SmallLds S;
+    const int t = (int)threadIdx.x, wv = t >> 6, lane = t & 63;
+    if (blockIdx.x > 0) {
+        const int xb = (int)blockIdx.x - 1;
+        if (xb < npk) {
+            const size_t q = (size_t)xb * kScanThreads + t;
+            if (q < PackLayout<true>::off[8]) pack_elem<true>(ps, pbuf, q);
+            return;
+        }
+        // input rows: eight lanes per 128-byte record (as k_decode)
+        const int g = (xb - npk) * (kScanThreads / 8) + (t >> 3), c = t & 7;
+        if (xb == npk && t < SSLA_MAX_BLOCKS) bd_out[t] = tab.d[t];
+        if (g >= E || c < 1 || c > SSLA_C1 / 4) return;
+        int b = 0;
+        for (int i = 1; i < G.nb; ++i)
+            if (g >= tab.d[i].offset) b = i;
+        const HybridInputRec* r = tab.d[b].ring + (g - tab.d[b].offset);
+        const float4 v = reinterpret_cast<const float4*>(r)[c];
+        const bool valid = r->x < G.W2 && r->y < G.H2;
+        reinterpret_cast<float4*>(X0 + (size_t)g * SSLA_C1)[c - 1] =
+            valid ? v : make_float4(0.f, 0.f, 0.f, 0.f);
+        return;
+    }
+    const int nk2 = G.nb * G.C2, nk3 = G.nb * G.C3, nv = E / kGP + 3;
+    const int rounds = (E + kScanThreads - 1) / kScanThreads;
+    // ---- keys of the records, their counts -----------------------------------
+    for (int i = t; i <= kScanThreads; i += kScanThreads) S.cur[i] = 0;
+    for (int i = t; i < kSmallWaves * (kScanThreads + 2); i += kScanThreads) (&S.wc[0][0])[i] = 0;
+    if (t < nv) S.hist[t] = 0;
+    if (t < 16) o.counts[t] = 0;
+    __syncthreads();
+    for (int g = t; g < E; g += kScanThreads) {
+        int b = 0;
+        for (int i = 1; i < G.nb; ++i)
+            if (g >= tab.d[i].offset) b = i;
+        const HybridInputRec* r = tab.d[b].ring + (g - tab.d[b].offset);
+        const HybridStrip& s = tab.d[b].strip;
+        const int x = r->x, y = r->y;
+        const bool valid = x < G.W2 && y < G.H2;
+        const bool own = valid && x >= s.owned_lo && x < s.owned_hi && y >= s.owned_y_lo &&
+                         y < s.owned_y_hi;
+        const int k = valid ? b * G.C2 + y * G.W2 + x : nk2;
+        o.cell2[g] = valid ? y * G.W2 + x : -1;
+        o.owner[g] = own ? 1 : 0;
+        S.key[g] = (unsigned short)(k | (own ? 0x8000 : 0));
+        atomicAdd(&S.cur[k], 1);
+    }
+    __syncthreads();
+    {
+        const int len = t < nk2 ? S.cur[t] : 0;
+        scan_keys(len, nk2, S.st, S.lds);
+        __syncthreads();
+        S.cur[t] = t <= nk2 ? S.st[t] : 0;
+        if (t == 0) S.cur[kScanThreads] = S.st[nk2];    // (keyless records, nk2 = kScanThreads)
+    }
+    __syncthreads();
+    // ---- stable sort: 1024 records a round, ranks as in k_rs_scatter ------------
+    for (int q = 0; q < rounds; ++q) {
+        const int g = q * kScanThreads + t;
+        const bool valid = g < E;
+        const int k = valid ? S.key[g] & 0x7fff : 0;
+        unsigned long long peers = __ballot(valid);
+        #pragma unroll
+        for (int b = 0; b < 11; ++b) {
+            const bool bit = (k >> b) & 1;
+            const unsigned long long m = __ballot(bit);
+            peers &= bit ? m : ~m;
+        }
+        const int rank = __popcll(peers & ((1ull << lane) - 1ull)), size = __popcll(peers);
+        const bool leader = valid && rank == 0;
+        if (leader) S.wc[wv][k] = (unsigned short)size;
+        __syncthreads();
+        if (valid) {
+            int pos = S.cur[k] + rank;
+            for (int w = 0; w < wv; ++w) pos += S.wc[w][k];
+            S.v2[pos] = (uint32_t)g;
+            S.k2[pos] = (uint32_t)k;
+            if constexpr (!ALL) {
+                o.vals2[pos] = (uint32_t)g;
+                o.keys2[pos] = (uint32_t)k;
+                o.sidx[g] = pos;
+            }
+        }
+        __syncthreads();
+        if (leader) {
+            atomicAdd(&S.cur[k], size);
+            S.wc[wv][k] = 0;
+        }
+        __syncthreads();
+    }
+    // ---- s2 keys: counters, pass-2 counts and offsets, pairs, groups -------------
+    {
+        int n2 = 0, np = 0;
+        if (t < nk2) {
+            const int b = t / G.C2, len = S.st[t + 1] - S.st[t];
+            unsigned char* td = tab.d[b].td2 + t % G.C2;
+            const unsigned c = *td;
+            S.old[t] = (unsigned char)c;
+            n2 = tdrop_passes(c, len, G.window);
+            *td = (unsigned char)((c + (unsigned)len) & 255u);
+            S.n2[t] = n2;
+            np = pair_count(t, G.C2, G.W2, G.H2, S.st);
+        }
+        int total;
+        const int off = block_exscan(n2, S.lds, &total);
+        const int go = block_exscan((np + kGP - 1) / kGP, S.lds, &total);
+        if (t < nk2) {
+            S.off[t] = off;
+            S.go[t] = go;
+        }
+        if constexpr (!ALL) {
+            if (t < nk2) {
+                o.st2[t] = S.st[t];
+                o.en2[t] = S.st[t + 1];
+                o.old2[t] = S.old[t];
+                o.n2[t] = n2;
+                o.off2[t] = off;
+            }
+            int n2all;
+            (void)block_exscan(n2, S.lds, &n2all);
+            if (t == 0) o.counts[0] = n2all;
+            if (o.have_head && t < nk3) {
+                o.last3[t] = -1;
+                o.cnt3[t] = 0;
+            }
+        }
+        scan_keys(np, nk2, S.pst, S.lds);
+    }
+    __syncthreads();
+    if constexpr (!ALL)
+        for (int i = t; i <= nk2; i += kScanThreads) o.pst2[i] = S.pst[i];
+    group_list_lds(nk2, S.pst, S.go, S.hist, S.start, S.lds, GroupTab{nv, o.glist2, o.counts + 6});
+    if constexpr (!ALL) return;
+    // ---- one record per thread from here ----------------------------------------
+    {
+        const bool take = tdrop2_at(t, E, S.k2, S.v2, (uint32_t)nk2, S.st, S.old, S.off, G.window,
+                                    o.pass2, o.list2);
+        pair_rank_at<true>(t, E, S.k2, S.v2, (uint32_t)nk2, G.C2, G.W2, G.H2, S.st, S.st + 1, S.pst,
+                     o.pent2, nullptr, take);
+    }
+    // ---- s3 keys: run lengths (in cur), starts, pass-3 counts and offsets ---------
+    // (the s2 pair starts, offsets and group tables are done with: their arrays
+    // take the s3 level's; st, n2, old stay for the s3 ranks)
+    __syncthreads();
+    {
+        int t3 = 0, n3 = 0;
+        if (t < nk3) {
+            const int b = t / G.C3, cell = t % G.C3;
+            const int s = b * G.C2 + 2 * (cell / G.W3) * G.W2 + 2 * (cell % G.W3);
+            t3 = S.n2[s] + S.n2[s + 1] + S.n2[s + G.W2] + S.n2[s + G.W2 + 1];
+            n3 = tdrop_passes(tab.d[b].td3[cell], t3, G.window);
+            S.last[t] = -1;
+            S.cnt[t] = 0;
+        }
+        if (t < nv) S.hist[t] = 0;
+        const int n2all = scan_keys(t3, nk3, S.cur, S.lds);
+        const int n3all = scan_keys(n3, nk3, S.pst, S.lds);
+        if (t < nk3) S.off[t] = S.pst[t];
+        if (t == 0) {
+            o.counts[0] = n2all;
+            o.counts[1] = n3all;
+        }
+        __syncthreads();
+        int np = 0;
+        if (t < nk3) np = pair_count(t, G.C3, G.W3, G.H3, S.cur);
+        int total;
+        const int go = block_exscan((np + kGP - 1) / kGP, S.lds, &total);
+        if (t < nk3) S.go[t] = go;
+        scan_keys(np, nk3, S.pst, S.lds);
+    }
+    // the pass-2 records in s3 order (ranks as in k_place3)
+    const int k2 = t < E ? (int)S.k2[t] : nk2;
+    if (k2 < nk2 && tdrop_pass(S.old[k2], (unsigned)(t - S.st[k2]), G.window)) {
+        const int i = t, k = k2;
+        const uint32_t g = S.v2[i];
+        const int b = k / G.C2, cell = k % G.C2, x = cell % G.W2, y = cell / G.W2;
+        const int x0 = x & ~1, y0 = y & ~1;
+        const int k3 = b * G.C3 + (y >> 1) * G.W3 + (x >> 1);
+        int rank = 0;
+        #pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int s = b * G.C2 + (y0 + (q >> 1)) * G.W2 + x0 + (q & 1);
+            const int lo = S.st[s];
+            const int r = s == k ? i - lo : lower_bound_u32(S.v2, lo, S.st[s + 1] - lo, g) - lo;
+            rank += tdrop_passes(S.old[s], r, G.window);
+        }
+        const int slot = S.cur[k3] + rank;
+        if (slot >= 0 && slot < kSmallAll) {              // (ranks are a permutation of [0, n))
+            S.k3[slot] = (uint32_t)k3;
+            S.v3[slot] = g;
+            o.key3g[g] = (uint32_t)k3;
+        }
+    }
+    __syncthreads();
+    group_list_lds(nk3, S.pst, S.go, S.hist, S.start, S.lds, GroupTab{nv, o.glist3, o.counts + 7});
+    const int n2all = S.cur[nk3];
+    {
+        const int p = t;
+        bool take = false;
+        if (p < n2all) {
+            const int k = (int)S.k3[p], g = (int)S.v3[p];
+            const int r = p - S.cur[k];
+            const unsigned c = tab.d[k / G.C3].td3[k % G.C3];
+            take = tdrop_pass(c, (unsigned)r, G.window);
+            o.pass3[g] = take ? 1 : 0;
+            if (take) {
+                o.list3[S.off[k] + tdrop_passes(c, r, G.window)] = g;
+                if (S.key[g] & 0x8000) {
+                    atomicMax(&S.last[k], g);
+                    atomicAdd(&S.cnt[k], 1);
+                }
+            }
+        }
+        pair_rank_at<true>(p, n2all, S.k3, S.v3, (uint32_t)nk3, G.C3, G.W3, G.H3, S.cur, S.cur + 1, S.pst,
+                     o.pent3, nullptr, take);
+    }
+    __syncthreads();
+    if (t < nk3) {
+        unsigned char* td = tab.d[t / G.C3].td3 + t % G.C3;
+        *td = (unsigned char)(((unsigned)*td + (unsigned)(S.cur[t + 1] - S.cur[t])) & 255u);
+        if (o.have_head) {
+            o.last3[t] = S.last[t];
+            o.cnt3[t] = S.cnt[t];
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1510,8 +1850,13 @@ k_pscan(const int* __restrict__ n_groups, int* __restrict__ ticket, unsigned tag
             }
         };
         // in flight: the next group's pairs, the group after it, the ticket after that
-        int tk = __builtin_amdgcn_readfirstlane(draw()), tk1 = __builtin_amdgcn_readfirstlane(draw());
-        int tk2 = draw();
+        int d0 = 0, d1 = 0, tk2 = 0;
+        if (lane == 0) {
+            d0 = atomicAdd(ticket, 1);
+            d1 = atomicAdd(ticket, 1);
+            tk2 = atomicAdd(ticket, 1);
+        }
+        int tk = __builtin_amdgcn_readfirstlane(d0), tk1 = __builtin_amdgcn_readfirstlane(d1);
         int4 gd = fetch(tk), gd1 = fetch(tk1);
         load_pairs(gd);
         for (int g = 0;; ++g) {
@@ -1695,6 +2040,10 @@ __device__ __forceinline__ double sum4_lanes(double v, int lane) {
 // one wave per SIMD).
 constexpr int kOutKS5 = 3, kOutKS6 = 3, kOutKS7 = 3;
 constexpr int kOutRT5 = 1, kOutRT6 = 1, kOutRT7 = 1;
+// A layer with at most two 16-record tiles per CU is a chain of load latencies
+// (27 items a wave in L4), so every delta gets a wave of its own (KS = 9); L7
+// keeps three, nine would spill.  At 300 records L4 22 -> 8 us, L6 18 -> 17.
+constexpr int kOutKSFew = 9, kOutKSFew7 = 3;
 
 template <int IN, int OUT, int RT, int KS, int WPS = 1>
 __global__ void __launch_bounds__(64 * KS, WPS)
@@ -1907,6 +2256,33 @@ __device__ __forceinline__ float quad_sum(float v) {
     return v;
 }
 
+// The prediction grid: a record's raw head row is published when it is the
+// last owned pass-3 record of its s3 cell (k_tdrop3), with the number of such
+// records added to the cell's version.  Each head kernel does it for the rows it
+// has just computed (a launch of its own for it cost the small drains 8 us).
+struct PredGrid {
+    const unsigned char* owner;
+    const uint32_t* key3_by_g;
+    const int *last, *count;
+    const BlockDesc* bd;
+    Geometry G;
+};
+
+__device__ __forceinline__ void pred_write(const PredGrid& p, int g, const float* v7) {
+    if (!p.owner[g]) return;
+    const uint32_t k = p.key3_by_g[g];
+    if (p.last[k] != g) return;
+    const int b = (int)k / p.G.C3, cell = (int)k % p.G.C3;
+    const HybridStrip& s = p.bd[b].strip;
+    const int sx = cell % p.G.W3, sy = cell / p.G.W3;
+    const int hx = sx - s.s3_owned_lo, hy = sy - s.s3_owned_y_lo;
+    const int w = s.s3_owned_hi - s.s3_owned_lo, h = s.s3_owned_y_hi - s.s3_owned_y_lo;
+    if (hx < 0 || hx >= w || hy < 0 || hy >= h) return;
+    const int idx = hy * w + hx;
+    publish_pred(p.bd[b].preds ? p.bd[b].preds + (size_t)idx * 7 : nullptr,
+                 p.bd[b].version ? p.bd[b].version + idx : nullptr, v7, (unsigned)p.count[k]);
+}
+
 // ---------------------------------------------------------------------------
 // head: raw [reg0..3, obj, cls0, cls1] for pass-3 records
 // (...celled.cuh:841-902).  One workgroup = 64 records (list order): their
@@ -1916,9 +2292,10 @@ __device__ __forceinline__ float quad_sum(float v) {
 // takes row 4s + l/16, column l%16 of step s); SiLU into LDS; then the
 // seven prediction dot products, four threads per record.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256)
+constexpr int kHeadThreads = 64 * 2 * SSLA_C3 / kMT;      // a wave per column tile
+__global__ void __launch_bounds__(kHeadThreads)
 k_head(const int* __restrict__ n_dev, const int* __restrict__ list,
-       const float* __restrict__ X, HeadPtrs hp, float* __restrict__ H7) {
+       const float* __restrict__ X, HeadPtrs hp, PredGrid pg, float* __restrict__ H7) {
     constexpr int C = SSLA_C3, XST = lds_stride(C), HST = 2 * C + 4, CT = 2 * C / kMT;
     __shared__ __align__(16) float xs[kTM * XST];
     __shared__ float hs[kTM * HST];           // [yc | yr] per record
@@ -1931,7 +2308,7 @@ k_head(const int* __restrict__ n_dev, const int* __restrict__ list,
     if (tid < kTM) rows[tid] = tid < cnt ? list[base + tid] : -1;
     __syncthreads();
     constexpr int C4 = C / 4;
-    for (int t = tid; t < kTM * C4; t += 256) {
+    for (int t = tid; t < kTM * C4; t += kHeadThreads) {
         const int r = t / C4, q = t - r * C4;
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
         if (rows[r] >= 0) v = reinterpret_cast<const float4*>(X)[(size_t)rows[r] * C4 + q];
@@ -1940,8 +2317,10 @@ k_head(const int* __restrict__ n_dev, const int* __restrict__ list,
     __syncthreads();
     const int lane = tid & 63, wv = tid >> 6, li = lane & 15, lk = lane >> 4;
     const int mtiles = (cnt + kMT - 1) / kMT;
-    // column tiles 0..5: cls conv, 6..11: reg conv; wave wv takes tiles wv, wv+4, wv+8
-    for (int ct = wv; ct < CT; ct += 4) {
+    // column tiles 0..5: cls conv, 6..11: reg conv, one per wave
+    {
+        const int ct = wv;
+        static_assert(kHeadThreads == 64 * CT, "a wave per column tile");
         const bool reg = ct >= CT / 2;
         const float* W = reg ? hp.reg_conv_W : hp.cls_conv_W;
         const float* bias = reg ? hp.reg_conv_b : hp.cls_conv_b;
@@ -1965,6 +2344,7 @@ k_head(const int* __restrict__ n_dev, const int* __restrict__ list,
     }
     __syncthreads();
     // predictions: record r = tid / 4, channels part, part + 4, ... (24 each)
+    if (tid >= 4 * kTM) return;
     const int r = tid >> 2, part = tid & 3;
     float o[7];
     #pragma unroll
@@ -1972,6 +2352,8 @@ k_head(const int* __restrict__ n_dev, const int* __restrict__ list,
     if (r < cnt) {
         const float* yc = &hs[r * HST];
         const float* yr = yc + C;
+        // (unrolled: a rolled loop waits for one channel's seven weights at a time)
+        #pragma unroll 6
         for (int i = part; i < C; i += 4) {
             #pragma unroll
             for (int k = 0; k < 4; ++k) o[k] = fmaf(hp.reg_pred_W[(size_t)i * 4 + k], yr[i], o[k]);
@@ -1985,10 +2367,13 @@ k_head(const int* __restrict__ n_dev, const int* __restrict__ list,
     if (r < cnt && part == 0) {
         float* out = H7 + (size_t)rows[r] * 7;
         #pragma unroll
-        for (int k = 0; k < 4; ++k) out[k] = o[k] + hp.reg_pred_b[k];
-        out[4] = o[4] + hp.obj_pred_b[0];
-        out[5] = o[5] + hp.cls_pred_b[0];
-        out[6] = o[6] + hp.cls_pred_b[1];
+        for (int k = 0; k < 4; ++k) o[k] += hp.reg_pred_b[k];
+        o[4] += hp.obj_pred_b[0];
+        o[5] += hp.cls_pred_b[0];
+        o[6] += hp.cls_pred_b[1];
+        #pragma unroll
+        for (int k = 0; k < 7; ++k) out[k] = o[k];
+        pred_write(pg, rows[r], o);
     }
 }
 
@@ -1998,7 +2383,7 @@ k_head(const int* __restrict__ n_dev, const int* __restrict__ list,
 // ...), the quad's partial sums added with two DPP moves.
 __global__ void __launch_bounds__(256)
 k_head_linear(const int* __restrict__ n_dev, const int* __restrict__ list,
-              const float* __restrict__ X, HeadPtrs hp, float* __restrict__ H7) {
+              const float* __restrict__ X, HeadPtrs hp, PredGrid pg, float* __restrict__ H7) {
     constexpr int C = SSLA_C3;
     const int n = *n_dev;
     const int base = blockIdx.x * kTM;
@@ -2022,41 +2407,21 @@ k_head_linear(const int* __restrict__ n_dev, const int* __restrict__ list,
     if (on && part == 0) {
         float* out = H7 + (size_t)g * 7;
         #pragma unroll
-        for (int k = 0; k < 7; ++k) out[k] = o[k] + hp.lin_b[k];
+        for (int k = 0; k < 7; ++k) {
+            o[k] += hp.lin_b[k];
+            out[k] = o[k];
+        }
+        pred_write(pg, g, o);
     }
-}
-
-__global__ void k_pred_write(const int* __restrict__ n_dev, const int* __restrict__ list,
-                             const unsigned char* __restrict__ owner,
-                             const uint32_t* __restrict__ key3_by_g,
-                             const int* __restrict__ last, const int* __restrict__ count,
-                             const BlockDesc* __restrict__ bd, Geometry G,
-                             const float* __restrict__ H7) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= *n_dev) return;
-    const int g = list[j];
-    if (!owner[g]) return;
-    const uint32_t k = key3_by_g[g];
-    if (last[k] != g) return;
-    const int b = (int)k / G.C3, cell = (int)k % G.C3;
-    const HybridStrip& s = bd[b].strip;
-    const int sx = cell % G.W3, sy = cell / G.W3;
-    const int hx = sx - s.s3_owned_lo, hy = sy - s.s3_owned_y_lo;
-    const int w = s.s3_owned_hi - s.s3_owned_lo, h = s.s3_owned_y_hi - s.s3_owned_y_lo;
-    if (hx < 0 || hx >= w || hy < 0 || hy >= h) return;
-    const int idx = hy * w + hx;
-    float v7[7];
-    #pragma unroll
-    for (int q = 0; q < 7; ++q) v7[q] = H7[(size_t)g * 7 + q];
-    publish_pred(bd[b].preds ? bd[b].preds + (size_t)idx * 7 : nullptr,
-                 bd[b].version ? bd[b].version + idx : nullptr, v7, (unsigned)count[k]);
 }
 
 // Output slots (...celled.cuh:1233-1247 conventions) and raw head rows.
 // Output slots (392 B = 49 eight-byte words) and head rows as coalesced
 // 8-byte stores: 32 records per 256-thread workgroup.
-constexpr int kEmitRec = 128;
+// (a small call: 8, so that its few records are not one workgroup's loop)
+constexpr int kEmitRec = 128, kEmitRecFew = 8;
 
+template <int RPB>
 __global__ void __launch_bounds__(256)
 k_emit(int E, const BlockDesc* __restrict__ bd, int nb,
        const int* __restrict__ cell2,
@@ -2067,11 +2432,11 @@ k_emit(int E, const BlockDesc* __restrict__ bd, int nb,
        int have_head) {
     constexpr int NW = (int)(sizeof(HybridS2S3OutputSlot) / 8);
     static_assert(sizeof(HybridS2S3OutputSlot) % 8 == 0 && SSLA_C3 % 2 == 0, "slot words");
-    __shared__ int sb[kEmitRec], sk[kEmitRec], sp2[kEmitRec], sp3[kEmitRec];
-    __shared__ unsigned char sfeat[kEmitRec], shead[kEmitRec];
-    const int g0 = blockIdx.x * kEmitRec;
+    __shared__ int sb[RPB], sk[RPB], sp2[RPB], sp3[RPB];
+    __shared__ unsigned char sfeat[RPB], shead[RPB];
+    const int g0 = blockIdx.x * RPB;
     const int t = threadIdx.x;
-    if (t < kEmitRec) {
+    if (t < RPB) {
         const int g = g0 + t;
         int b = 0, k = -1, q2 = -2, q3 = -2;
         bool feat = false, head = false;
@@ -2091,7 +2456,7 @@ k_emit(int E, const BlockDesc* __restrict__ bd, int nb,
         sfeat[t] = feat; shead[t] = head;
     }
     __syncthreads();
-    for (int j = t; j < kEmitRec * NW; j += 256) {
+    for (int j = t; j < RPB * NW; j += 256) {
         const int r = j / NW, w = j - r * NW;
         const int k = sk[r];
         HybridS2S3OutputSlot* out = k >= 0 ? bd[sb[r]].out : nullptr;
@@ -2105,7 +2470,7 @@ k_emit(int E, const BlockDesc* __restrict__ bd, int nb,
             reinterpret_cast<float2*>(out[k].s3_feat)[w - 1] = f;
         }
     }
-    for (int j = t; j < kEmitRec * 7; j += 256) {
+    for (int j = t; j < RPB * 7; j += 256) {
         const int r = j / 7, c = j - r * 7;
         const int k = sk[r];
         float* ho = k >= 0 ? bd[sb[r]].head_out : nullptr;
@@ -2334,12 +2699,15 @@ inline unsigned grid1(long long n, int bs) { return (unsigned)((n + bs - 1) / bs
 struct CallEnd {
     Workspace& w;
     hipStream_t st;
+    bool side = false;         // the call has launched on the side stream
     bool ended = false;
     void finish() {
         if (ended) return;
         ended = true;
-        (void)hipEventRecord(w.side_done, w.side);
-        (void)hipStreamWaitEvent(st, w.side_done, 0);
+        if (side) {
+            (void)hipEventRecord(w.side_done, w.side);
+            (void)hipStreamWaitEvent(st, w.side_done, 0);
+        }
         (void)hipEventRecord(w.done, st);
     }
     ~CallEnd() { finish(); }
@@ -2514,6 +2882,11 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
     const PackSrc psrc = pack_setup<true>(cfg->layers[0], w.packed, &w.pk);
     const PackedWeights& pk = w.pk;
     MARK();
+    const LayerWeightsS2S3* L = cfg->layers[0];
+    const bool small = E <= kSmallRec && nk2 <= (uint32_t)kScanThreads;
+    const bool small_all = small && E <= kSmallAll;      // the s3 ordering too
+    uint32_t *K2 = w.ka, *V2 = w.va, *K3 = w.kb, *V3 = w.vb;
+    hipStream_t s3 = w.side;
     // per-call fills: run bounds of the s2 keys (k_runs writes those that
     // occur), the list and group counters, the prediction-grid writers
     // the group-count bound of this call's cells (see ensure_workspace), and
@@ -2533,6 +2906,19 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
             f.v[i] = val[i];
         }
     }
+    if (small) {
+        const int npk = (int)((PackLayout<true>::off[8] + kScanThreads - 1) / kScanThreads);
+        const SmallOut o{w.cell2, w.owner, w.pass2, w.pass3, w.list2, w.list3, w.counts, w.last3,
+                         w.cnt3, w.key3g, w.pent2, w.pent3, w.glist, w.glist3, have_head ? 1 : 0,
+                         K2, V2, w.sidx, w.st2, w.en2, w.pst2, w.n2, w.off2, w.old2};
+        const dim3 grid(1 + npk + grid1(E, kScanThreads / 8));
+        if (small_all)
+            hipLaunchKernelGGL(k_small_order<true>, grid, dim3(kScanThreads), 0, st, E, tab, w.bd, G,
+                               w.X0, o, psrc, w.packed, npk);
+        else
+            hipLaunchKernelGGL(k_small_order<false>, grid, dim3(kScanThreads), 0, st, E, tab, w.bd, G,
+                               w.X0, o, psrc, w.packed, npk);
+    } else {
     // ---- decode (and the fills); stable radix sort of the records by s2 key --
     {
         const int ndec = (int)grid1(E, kDecRec), fblk = (int)grid1(std::max<int>(std::max<int>((int)nk2, 16), nv), 256);
@@ -2569,10 +2955,10 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
         vout = v2;
     }
     // the sorted s2 order, and the buffers the s3 order is placed in
-    uint32_t* const K2 = kin;
-    uint32_t* const V2 = vin;
-    uint32_t* const K3 = kout;
-    uint32_t* const V3 = vout;
+    K2 = kin;
+    V2 = vin;
+    K3 = kout;
+    V3 = vout;
     // ---- counters, tdrop_s2, the pass-2 list, s2 pair and group tables -----
     if (passes == 1 && nk2 <= (uint32_t)kScanThreads) {
         // the one pass's histogram holds the run bounds: the key tables and
@@ -2600,16 +2986,20 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
                                w.pcnt, w.pst2, (int*)nullptr, w.goff2, w.n2, w.off2, w.counts + 0,
                                KeyHist{}, GroupTab{});
     }
-    {
+    }
+    if (!small_all) {
         const unsigned nbr = grid1(E, 256);
-        hipLaunchKernelGGL(k_s2_tables, dim3(nbr + (gt2 ? 0u : grid1(nk2, 256))), dim3(256), 0, st, E,
-                           (int)nbr, K2, V2, nk2, G.C2, G.W2, G.H2, w.st2, w.en2, w.pst2, w.old2,
-                           w.off2, G.window, w.pass2, w.list2, w.pent2, w.gcnt, w.gend, w.ghist, w.gw);
+#define S2_TABLES(SMALL)                                                                              \
+    hipLaunchKernelGGL(k_s2_tables<SMALL>, dim3(nbr + (gt2 ? 0u : grid1(nk2, 256))), dim3(256), 0, st, E, \
+                       (int)nbr, K2, V2, nk2, G.C2, G.W2, G.H2, w.st2, w.en2, w.pst2, w.old2, w.off2,  \
+                       G.window, w.pass2, w.list2, w.pent2, w.gcnt, w.gend, w.ghist, w.gw)
+        if (E <= kSmallRec) S2_TABLES(true);
+        else S2_TABLES(false);
+#undef S2_TABLES
         if (!gt2)
             hipLaunchKernelGGL(k_group_order, dim3(1), dim3(kScanThreads), 0, st, (int)nk2, nv, w.pst2,
                                w.goff2, w.gcnt, w.gend, w.ghist, w.gw, w.gstart, w.gbase, w.glist,
                                w.counts + 6);
-    }
     // The s3 ordering needs only the s2 order, pass2 and the old counters, so
     // it runs on the side stream while L4 and L5 run here; L6 waits for it.
     // Its launches are sized by E; the pass-2 count stays on the device.  Its
@@ -2617,10 +3007,10 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
     // start beside the projection rather than beside the latency-bound parts
     // that follow it.
     HIPCHK(hipEventRecord(w.s2_ordered, st));
-    hipStream_t s3 = w.side;
+    end.side = true;
     HIPCHK(hipStreamWaitEvent(s3, w.s2_ordered, 0));
+    }
     MARK();
-    const LayerWeightsS2S3* L = cfg->layers[0];
     // The pass-2 and pass-3 counts stay on the device; the launches over their
     // lists are sized by bounds the host has.  A cell's L records in a row take
     // at most L P / 256 + 2 passes of the tdrop gate, P = ceil(256 / window)
@@ -2663,13 +3053,25 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
     } while (0)
     // ---- L4: 24 -> 48, all records ----------------------------------------
     PSCAN(SSLA_C1, SSLA_C2, true, 0, 2, 6, w.glist, true, w.X0, G.C2, gridS4);
-    hipLaunchKernelGGL((k_outt<SSLA_C1, SSLA_C2, 2, 1, 3>), dim3(grid1(E, 32)), dim3(64), 0, st, E,
-                       no_count, no_list, w.X0, w.cell2, 0, G.W2, G.W2, G.H2, w.HR, pk.po[0],
-                       L[0].ln_gamma, L[0].ln_beta, w.X1);
+    const auto few = [&](int n) { return grid1(n, 16) <= 2 * cus; };
+#define OUTT(LI, IN, OUT, RT, KS, WPS, KSF, N, COUNT, LIST, XIN, SH, WL, HL, XOUT)                           \
+    do {                                                                                            \
+        if (few(N))                                                                                 \
+            hipLaunchKernelGGL((k_outt<IN, OUT, 1, KSF>), dim3(grid1(N, 16)),                        \
+                               dim3(64 * KSF), 0, st,       E, COUNT, LIST, XIN, w.cell2, SH, G.W2,  \
+                               WL, HL, w.HR, pk.po[LI], L[LI].ln_gamma, L[LI].ln_beta, XOUT);       \
+        else                                                                                        \
+            hipLaunchKernelGGL((k_outt<IN, OUT, RT, KS, WPS>), dim3(grid1(N, 16 * RT)), dim3(64 * KS), \
+                               0, st, E, COUNT, LIST, XIN, w.cell2, SH, G.W2, WL, HL, w.HR,         \
+                               pk.po[LI], L[LI].ln_gamma, L[LI].ln_beta, XOUT);                     \
+    } while (0)
+    const int *const n2_dev = w.counts + 0, *const n3_dev = w.counts + 1;
+    OUTT(0, SSLA_C1, SSLA_C2, 2, 1, 3, kOutKSFew, E, no_count, no_list, w.X0, 0, G.W2, G.H2, w.X1);
     MARK();
     // ---- [side] the s3 record order, tdrop_s3, s3 pair and group tables ---
     // (enqueued after L4's launches: the host needs a few microseconds per
     // launch, and L4 keeps the device busy meanwhile)
+    if (!small_all) {
     hipLaunchKernelGGL(k_keys3a, dim3(grid1(nk3, 256)), dim3(256), 0, s3, nk3, G, w.n2, w.bd,
                        w.t3, w.n3);
     hipLaunchKernelGGL((k_keyscan<false, false>), dim3(1), dim3(kScanThreads), 0, s3, (int)nk3, w.t3,
@@ -2697,54 +3099,52 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
                            w.goff3, w.gcnt3, w.gend3, w.ghist3, w.gw3, w.gstart3, w.gbase3, w.glist3,
                            w.counts + 7);
     }
-    hipLaunchKernelGGL(k_pair_rank, dim3(grid1(nmax2, 256)), dim3(256), 0, s3, E,
-                       (const int*)(w.counts + 0), K3, V3, nk3, G.C3, G.W3, G.H3, w.st3, w.en3,
-                       w.pst3, w.pent3, w.pass3);
+#define PAIR_RANK3(SMALL)                                                                             \
+    hipLaunchKernelGGL(k_pair_rank<SMALL>, dim3(grid1(nmax2, 256)), dim3(256), 0, s3, E, n2_dev, K3, V3, nk3, \
+                       G.C3, G.W3, G.H3, w.st3, w.en3, w.pst3, w.pent3, w.pass3)
+    if (nmax2 <= kSmallRec) PAIR_RANK3(true);
+    else PAIR_RANK3(false);
+#undef PAIR_RANK3
     HIPCHK(hipEventRecord(w.s3_ordered, s3));
+    }
     HIPCHK(hipGetLastError());
     // ---- L5: 48 -> 48, state for all records, output for pass2 ---------------
     PSCAN(SSLA_C2, SSLA_C2, true, 1, 2, 6, w.glist, false, w.X1, G.C2, gridS4);
-    hipLaunchKernelGGL((k_outt<SSLA_C2, SSLA_C2, kOutRT5, kOutKS5>), dim3(grid1(nmax2, 16 * kOutRT5)),
-                       dim3(64 * kOutKS5), 0, st, E, (const int*)(w.counts + 0), w.list2, w.X1,
-                       w.cell2, 0, G.W2, G.W2, G.H2, w.HR, pk.po[1], L[1].ln_gamma, L[1].ln_beta,
-                       w.X2);
+    OUTT(1, SSLA_C2, SSLA_C2, kOutRT5, kOutKS5, 1, kOutKSFew, nmax2, n2_dev, w.list2, w.X1, 0, G.W2, G.H2, w.X2);
     MARK();
     // ---- L6: 48 -> 96, pass2 records ------------------------------------------
-    HIPCHK(hipStreamWaitEvent(st, w.s3_ordered, 0));
+    if (!small_all) HIPCHK(hipStreamWaitEvent(st, w.s3_ordered, 0));
     PSCAN(SSLA_C2, SSLA_C3, false, 2, 3, 7, w.glist3, true, w.X2, G.C3, gridS6);
-    hipLaunchKernelGGL((k_outt<SSLA_C2, SSLA_C3, kOutRT6, kOutKS6>), dim3(grid1(nmax2, 16 * kOutRT6)),
-                       dim3(64 * kOutKS6), 0, st, E, (const int*)(w.counts + 0), w.list2, w.X2,
-                       w.cell2, 1, G.W2, G.W3, G.H3, w.HR, pk.po[2], L[2].ln_gamma, L[2].ln_beta,
-                       w.X3);
+    OUTT(2, SSLA_C2, SSLA_C3, kOutRT6, kOutKS6, 1, kOutKSFew, nmax2, n2_dev, w.list2, w.X2, 1, G.W3, G.H3, w.X3);
     MARK();
     // ---- L7: 96 -> 96, state for pass2, output for pass3 ----------------------
     PSCAN(SSLA_C3, SSLA_C3, false, 3, 3, 7, w.glist3, false, w.X3, G.C3, gridS6);
-    hipLaunchKernelGGL((k_outt<SSLA_C3, SSLA_C3, kOutRT7, kOutKS7>), dim3(grid1(nmax3, 16 * kOutRT7)),
-                       dim3(64 * kOutKS7), 0, st, E, (const int*)(w.counts + 1), w.list3, w.X3,
-                       w.cell2, 1, G.W2, G.W3, G.H3, w.HR, pk.po[3], L[3].ln_gamma, L[3].ln_beta,
-                       w.X4);
+    OUTT(3, SSLA_C3, SSLA_C3, kOutRT7, kOutKS7, 1, kOutKSFew7, nmax3, n3_dev, w.list3, w.X3, 1, G.W3, G.H3, w.X4);
     MARK();
     HIPCHK(hipGetLastError());
     // ---- head ------------------------------------------------------------------
     if (have_head) {
         const HeadPtrs hp = head_ptrs(cfg);
+        const PredGrid pg{w.owner, w.key3g, w.last3, w.cnt3, w.bd, G};
         if (head == kHeadYolox)
-            hipLaunchKernelGGL(k_head, dim3(tiles3), dim3(256), 0, st, (const int*)(w.counts + 1),
-                               w.list3, w.X4, hp, w.H7);
+            hipLaunchKernelGGL(k_head, dim3(tiles3), dim3(kHeadThreads), 0, st, (const int*)(w.counts + 1),
+                               w.list3, w.X4, hp, pg, w.H7);
         else
             hipLaunchKernelGGL(k_head_linear, dim3(tiles3), dim3(256), 0, st,
-                               (const int*)(w.counts + 1), w.list3, w.X4, hp, w.H7);
-        hipLaunchKernelGGL(k_pred_write, dim3(grid1(nmax3, 256)), dim3(256), 0, st,
-                           (const int*)(w.counts + 1), w.list3, w.owner, w.key3g, w.last3,
-                           w.cnt3, w.bd, G, w.H7);
+                               (const int*)(w.counts + 1), w.list3, w.X4, hp, pg, w.H7);
     }
     MARK();
-    hipLaunchKernelGGL(k_emit, dim3(grid1(E, kEmitRec)), dim3(256), 0, st, E, w.bd, nb, w.cell2, w.owner,
-                       w.pass2, w.pass3, w.X4, w.H7, have_head ? 1 : 0);
+    if (grid1(E, kEmitRec) < cus)
+        hipLaunchKernelGGL(k_emit<kEmitRecFew>, dim3(grid1(E, kEmitRecFew)), dim3(256), 0, st, E, w.bd, nb,
+                           w.cell2, w.owner, w.pass2, w.pass3, w.X4, w.H7, have_head ? 1 : 0);
+    else
+        hipLaunchKernelGGL(k_emit<kEmitRec>, dim3(grid1(E, kEmitRec)), dim3(256), 0, st, E, w.bd, nb, w.cell2,
+                           w.owner, w.pass2, w.pass3, w.X4, w.H7, have_head ? 1 : 0);
     HIPCHK(hipGetLastError());
     MARK();
 #undef MARK
 #undef PSCAN
+#undef OUTT
     end.finish();
     if (phase_ms) {
         // this call's events join the pending ones (read below when sync is
