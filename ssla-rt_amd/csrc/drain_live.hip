@@ -71,7 +71,7 @@ struct LiveDesc {
     float* hidden[4];
     unsigned char* td2;
     unsigned char* td3;
-    float* scratch;                     // LP rows of 3*96 floats
+    float* scratch;                     // LP + 1 rows of 3*96 floats (the last: never read)
     HybridS2S3OutputSlot* out;          // batch mode
     float* head_out;                    // batch mode
     unsigned long long* batch_clk;      // batch mode
@@ -133,7 +133,7 @@ struct alignas(16) Lds {
     int dev[kPatch][LB];                 // records with a pair at delta
     int devo[kPatch][LB];                // ... that are output records of the layer
     int ol[LB];                          // output records of the current layer
-    int nlead, nout, bsize, flag, prof_on;
+    int nlead, nout, nset, bsize, flag, prof_on;
     unsigned long long t_pop, tprev;
     unsigned long long prof[NPROF];
 };
@@ -358,57 +358,63 @@ __device__ __forceinline__ void build_pairs(SL& S, int B, const unsigned char* s
 // whole (delta, column tile) items and keeps the tile's IN x 16 weights in
 // registers across its row tiles, and loads its next item's weights while
 // the current item runs.
-//   A operand: lane (i, k) = (lane % 16, lane / 16) holds row i, k
-//   B operand: lane holds column i, k;  D: lane holds rows 4k..4k+3, column i
-template <int IN, int OUT>
-struct ProjTile : ProjPack<IN, OUT> {
-    using ProjPack<IN, OUT>::T;
-    using ProjPack<IN, OUT>::TQ;
-    using ProjPack<IN, OUT>::KS;
-    using ProjPack<IN, OUT>::NC;
-    static __device__ __forceinline__ void run(Lds& S, int it, int li, int lk, const float* b,
-                                               float* __restrict__ scratch) {
-        const int d = it / T, t = it - d * T;
-        const bool qt = t < TQ;
-        const int n = qt ? S.dcnto[d] : S.dcnt[d];
-        const int* list = qt ? S.devo[d] : S.dev[d];
-        const int col = t * MT + li;
-        const float* X = &S.X[0][0];
-        for (int m0 = 0; m0 < n; m0 += MT) {
-            const int xr = list[min(m0 + li, n - 1)] * XS + lk;
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            #pragma unroll
-            for (int s = 0; s < KS; ++s)
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(X[xr + s * 4], b[s], acc, 0, 0, 0);
-            #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int rr = m0 + 4 * lk + r;
-                if (rr < n) gstore(scratch + (size_t)S.pidx[list[rr]][d] * NC + col, acc[r]);
-            }
-        }
-    }
-};
+// kProjAhead items' weights are in flight, v and g items first; the q items run
+// only when the layer has output records.  No load sits behind a branch (items
+// past the last repeat it) and an item has a fixed number of stores (an absent
+// record's row goes to the spare pair row LP), so a wait covers only the item it
+// is for.  (With a loop over row tiles the compiler waited for every load in
+// flight, the prefetched item included, before each item.)  An item whose delta
+// has no pair skips its products.  MTL: 16-record tiles of the layer's records.
+// Per batch of 8 (16 streams) L4..L7 took 9.9 / 9.6 / 12.9 / 16.4 us with the loop
+// and 7.1 / 9.0 / 10.4 / 13.6 now; the weights at a CU's 64 B a clock would take
+// 0.5 / 1.1 / 2.2 / 4.3.  Five items ahead (L4..L6) were 5% slower.
+//   A operand: the weights, lane (i, k) = (lane % 16, lane / 16) holds channel i
+//   B operand: the records;  D: lane holds channels 4k..4k+3 of record i, one
+//   float4 of its row
+constexpr int kProjAhead = 3;
 
-template <int IN, int OUT>
+template <int IN, int OUT, int MTL>
 __device__ __forceinline__ void phase_proj(Lds& S, const float* __restrict__ pp,
                                            float* __restrict__ scratch) {
-    using P = ProjTile<IN, OUT>;
-    static_assert(OUT % MT == 0 && IN % 4 == 0, "tile shapes");
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    using P = ProjPack<IN, OUT>;
+    constexpr int T = P::T, TQ = P::TQ, KS = P::KS, NC = P::NC;
+    constexpr int NVG = kPatch * 2 * TQ;            // v, g items; then the q items
+    static_assert(T == 3 * TQ && P::N == NVG + kPatch * TQ, "q, v, g column tiles");
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int li = lane & 15, lk = lane >> 4;
-    // two items in flight per wave: the next item's weights load while the
-    // current item's tiles run
-    float b0[P::KS4 * 4], b1[P::KS4 * 4];
-    int it = wv;
-    if (it < P::N) P::load(pp, it, lane, b0);
-    while (it < P::N) {
-        const int i1 = it + NW, i2 = i1 + NW;
-        if (i1 < P::N) P::load(pp, i1, lane, b1);
-        P::run(S, it, li, lk, b0, scratch);
-        if (i1 >= P::N) break;
-        if (i2 < P::N) P::load(pp, i2, lane, b0);
-        P::run(S, i1, li, lk, b1, scratch);
-        it = i2;
+    const int ni = __builtin_amdgcn_readfirstlane(S.nout > 0 ? P::N : NVG);
+    // item k of the wave: its place in the packed copy
+    auto item = [&](int k) {
+        const int j = min(wv + k * NW, ni - 1);
+        return j < NVG ? j / (2 * TQ) * T + TQ + j % (2 * TQ) : (j - NVG) / TQ * T + (j - NVG) % TQ;
+    };
+    float b[kProjAhead][P::KS4 * 4];
+    #pragma unroll
+    for (int k = 0; k < kProjAhead; ++k) P::load(pp, item(k), lane, b[k]);
+    const float* X = &S.X[0][0];
+    #pragma unroll 1
+    for (int k0 = 0; wv + k0 * NW < ni; k0 += kProjAhead) {
+        #pragma unroll
+        for (int k = 0; k < kProjAhead; ++k) {
+            const int it = item(k0 + k);
+            const int d = it / T, t = it - d * T;
+            const bool qt = t < TQ;
+            const int n = __builtin_amdgcn_readfirstlane(qt ? S.dcnto[d] : S.dcnt[d]);
+            const int* list = qt ? S.devo[d] : S.dev[d];
+            #pragma unroll
+            for (int m = 0; m < MTL && n > 0; ++m) {
+                const bool ok = m * MT + li < n;
+                const int rec = ok ? list[m * MT + li] : 0;
+                const int p = S.pidx[rec][d];
+                const float* xr = X + rec * XS + lk;
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                #pragma unroll
+                for (int s = 0; s < KS; ++s)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(b[k][s], xr[s * 4], acc, 0, 0, 0);
+                *(SSLA_GLOBAL f32x4*)(scratch + (size_t)(ok ? p : LP) * NC + t * MT + 4 * lk) = acc;
+            }
+            P::load(pp, item(k0 + k + kProjAhead), lane, b[k]);
+        }
     }
 }
 
@@ -455,72 +461,68 @@ __device__ __forceinline__ void phase_recur(Lds& S, float* __restrict__ hidden,
     }
 }
 
-// One (column tile, K part) item of the contraction below: B operand loads
-// (the part's weights, one register per 4-row step) and the MFMA chain over
-// the staged rows, leaving the partial tile in S.PK[part].
-template <int IN, int OUT>
-struct OutTile : OutPack<IN, OUT> {
-    using OutPack<IN, OUT>::SPER;
-    using OutPack<IN, OUT>::STEPS;
-    static __device__ __forceinline__ void run(Lds& S, int it, int li, int lk, const float* b) {
-        const int nt = it / KSPL, ks = it - nt * KSPL;
-        const int col = nt * MT + li;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        #pragma unroll
-        for (int j = 0; j < SPER; ++j) {
-            const int s = min(ks * SPER + j, STEPS - 1);  // past the end b is 0
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(S.QH[li][s * 4 + lk], b[j], acc, 0, 0, 0);
-        }
-        #pragma unroll
-        for (int r = 0; r < 4; ++r) S.PK[ks][4 * lk + r][col] = acc[r];
-    }
-};
-
 // O: Y[e] = sum_delta goW[delta]^T qh(e, delta) + residual for the output
 // records S.ol[0, S.nout), 16 records at a time, as one MFMA contraction
 // over K = 9*OUT (+ IN): each record's row holds its nine q*h rows (zeros
 // where the patch cell is out of bounds) and, with input_proj, its input;
 // B is goW (9*OUT x OUT, delta-major) followed by input_proj.  Waves own
 // (column tile, K part) items with the part's weights in registers; the
-// parts are added in order.
+// parts are added in order.  The rows are staged four floats at a time with every
+// load in flight at once, behind the first items' weights (per batch of 8: L4 5.1
+// -> 3.8 us, L6 10.6 -> 7.1).
 template <int IN, int OUT>
 __device__ __forceinline__ void phase_out(Lds& S, const float* __restrict__ po,
                                           const float* __restrict__ scratch) {
-    using O = OutTile<IN, OUT>;
-    constexpr int NC = 3 * OUT;
-    static_assert(O::KT <= QS, "contraction row");
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int li = lane & 15, lk = lane >> 4;
+    using O = OutPack<IN, OUT>;
+    constexpr int NC = 3 * OUT, SPER = O::SPER, NIT = O::N / NW, AH = NIT > 3 ? 2 : NIT;
+    constexpr int K4 = O::KT / 4, O4 = OUT / 4, SIT = (MT * K4 + LT - 1) / LT;
+    static_assert(O::KT <= QS && QS % 4 == 0 && O::N % NW == 0 && NIT % AH == 0, "contraction row, items");
     const int no = S.nout;
     for (int c0 = 0; c0 < no; c0 += MT) {
+        // (formed per chunk: the compiler otherwise keeps every row's and
+        // item's address across the chunks, in scratch)
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const int li = lane & 15, lk = lane >> 4;
         const int m = min(MT, no - c0);
-        for (int t = tid; t < MT * O::KT; t += LT) {
-            const int r = t / O::KT, k = t - r * O::KT;
-            float v = 0.f;
-            if (r < m) {
-                const int e = S.ol[c0 + r];
-                if (k < O::KQ) {
-                    const int d = k / OUT, i = k - d * OUT;
-                    const int p = S.pidx[e][d];
-                    if (p >= 0) v = gload(scratch + (size_t)p * NC + i);
-                } else {
-                    v = S.X[e][k - O::KQ];
-                }
-            }
-            S.QH[r][k] = v;
+        // the first items' weights, on their way while the rows are staged
+        float b[AH][O::SP4 * 4];
+        #pragma unroll
+        for (int k = 0; k < AH; ++k) O::load(po, wv + k * NW, lane, b[k]);
+        // the rows, four floats at a time, every load issued before the first
+        // is used (an absent pair reads row 0 and is zeroed)
+        f32x4 v[SIT];
+        #pragma unroll
+        for (int j = 0; j < SIT; ++j) {
+            const int t = min(tid + j * LT, MT * K4 - 1), r = t / K4, k = t - r * K4;
+            const int d = min(k / O4, kPatch - 1), i = k - d * O4;
+            const int e = S.ol[c0 + min(r, m - 1)];
+            const int p = r < m ? S.pidx[e][d] : -1;
+            const bool in = O::IP && k >= kPatch * O4;        // the input's columns
+            const f32x4 h = *(const SSLA_GLOBAL f32x4*)(scratch + (size_t)max(p, 0) * NC + (in ? 0 : 4 * i));
+            const f32x4 x = *(const f32x4*)&S.X[e][in ? 4 * (k - kPatch * O4) : 0];
+            #pragma unroll
+            for (int q = 0; q < 4; ++q) v[j][q] = in ? (r < m ? x[q] : 0.f) : p >= 0 ? h[q] : 0.f;
+        }
+        #pragma unroll
+        for (int j = 0; j < SIT; ++j) {
+            const int t = tid + j * LT, r = t / K4, k = t - r * K4;
+            if (t < MT * K4) *(f32x4*)&S.QH[r][4 * k] = v[j];
         }
         __syncthreads();
-        float b0[O::SP4 * 4], b1[O::SP4 * 4];
-        int it = wv;
-        if (it < O::N) O::load(po, it, lane, b0);
-        while (it < O::N) {
-            const int i1 = it + NW, i2 = i1 + NW;
-            if (i1 < O::N) O::load(po, i1, lane, b1);
-            O::run(S, it, li, lk, b0);
-            if (i1 >= O::N) break;
-            if (i2 < O::N) O::load(po, i2, lane, b0);
-            O::run(S, i1, li, lk, b1);
-            it = i2;
+        #pragma unroll
+        for (int k = 0; k < NIT; ++k) {
+            const int it = wv + k * NW, nt = it / KSPL, ks = it - nt * KSPL;
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+            #pragma unroll
+            for (int j = 0; j < SPER; ++j) {
+                const int s = min(ks * SPER + j, O::STEPS - 1);     // past the end b is 0
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(S.QH[li][s * 4 + lk], b[k % AH][j], acc, 0, 0, 0);
+            }
+            #pragma unroll
+            for (int r = 0; r < 4; ++r) S.PK[ks][4 * lk + r][nt * MT + li] = acc[r];
+            if (k + AH < NIT) O::load(po, it + AH * NW, lane, b[k % AH]);
         }
         __syncthreads();
         for (int t = tid; t < m * OUT; t += LT) {
@@ -547,7 +549,11 @@ __device__ __forceinline__ void batch_layer(Lds& S, int B, const unsigned char* 
         const unsigned long long lt = (1ull << tid) - 1ull;
         const unsigned long long bal = __ballot(o);
         if (o) S.ol[__popcll(bal & lt)] = tid;
-        if (tid == 0) S.nout = __popcll(bal);
+        const unsigned long long in = __ballot(tid < B && set[tid]);
+        if (tid == 0) {
+            S.nout = __popcll(bal);
+            S.nset = __popcll(in);
+        }
         #pragma unroll
         for (int d = 0; d < kPatch; ++d) {
             const bool has = o && S.pidx[tid][d] >= 0;
@@ -557,7 +563,13 @@ __device__ __forceinline__ void batch_layer(Lds& S, int B, const unsigned char* 
         }
     }
     __syncthreads();
-    phase_proj<IN, OUT>(S, pp, scratch);
+    // no record of the batch enters the layer (few pass tdrop_s2): nothing to do
+    if (S.nset == 0) {
+        __syncthreads();
+        return;
+    }
+    if (S.nset <= MT) phase_proj<IN, OUT, 1>(S, pp, scratch);
+    else phase_proj<IN, OUT, 2>(S, pp, scratch);
     __syncthreads();
     mark(S, slot + 0);
     phase_recur<OUT>(S, hidden, scratch, outm);
@@ -2034,7 +2046,7 @@ k_group(const LiveDesc* __restrict__ ld, LiveWeights W, Geometry G, GroupArgs ga
         }                                                                     \
     } while (0)
 
-size_t scratch_floats() { return (size_t)LP * NCMAX; }
+size_t scratch_floats() { return (size_t)(LP + 1) * NCMAX; }
 
 // batch-mode workspace: per-block scratch rows + the device block table
 std::mutex g_bmu;
@@ -2190,14 +2202,14 @@ int batch_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
 namespace {
 
 // Device memory the batch kernel uses beyond its inputs and outputs, for up
-// to kNaMaxBlocks blocks: each block's pair rows (LP x NCMAX floats), the
+// to kNaMaxBlocks blocks: each block's pair rows (LP + 1 rows of NCMAX floats), the
 // fragment-order weight copy and the block table.  One array per device,
 // held until the process ends; every call on a device shares it, so calls
 // that overlap on one device race.  Nothing in it has to start at zero: a
 // batch writes every pair row it reads, and each call rewrites the weight
 // copy and the block table before its kernel runs.
 constexpr int kNaMaxBlocks = SSLA_MAX_BLOCKS;
-constexpr size_t kNaRowFloats = (size_t)LP * NCMAX;                     // per block
+constexpr size_t kNaRowFloats = (size_t)(LP + 1) * NCMAX;               // per block
 constexpr size_t kNaPackOff = sizeof(float) * kNaRowFloats * kNaMaxBlocks;
 constexpr size_t kNaDescOff =
     (kNaPackOff + sizeof(float) * PackLayout<false>::off[8] + 255) & ~size_t(255);
