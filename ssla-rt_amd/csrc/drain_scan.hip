@@ -1427,10 +1427,10 @@ k_small_order(int E, BlockTable tab, BlockDesc* __restrict__ bd_out, Geometry G,
 //   rows (two teams of 3 waves, every other group each)   thread (sub, channel)
 //     takes kPSRows consecutive rows into registers, which frees the LDS buffer
 //     for the group after the next, and composes their map h -> A h + B (a cell's
-//     first pair has its cell's stored state folded in: A = 0); with its start
-//     state it replays them, writes h at row 9 g + d where the pair's record
-//     needs the layer's output (a record's nine rows are contiguous for its
-//     contraction), and stores the state of a cell's last pair;
+//     first pair has its cell's stored state folded in and drops what came
+//     before); with its start state it replays them, writes h at row 9 g + d where
+//     the pair's record needs the layer's output (a record's nine rows are
+//     contiguous for its contraction), and stores the state of a cell's last pair;
 //   chain (1 wave)   composes the group's map and finds its start state: none
 //     needed for a group that begins with a cell's first pair, else by looking
 //     back over the cell's earlier groups -- the nearest one whose end state is
@@ -1567,6 +1567,7 @@ constexpr int kPSStride = 2 * kPSC + 4;     // LDS row [v | sigmoid(g)]: 16 rows
 constexpr int kPSTiles = kPatch + (kGP - kPatch) / 16;       // most tiles of a group
 constexpr int kPSMask = (kGP + 63) / 64;    // 64-pair blocks of a group
 constexpr int kPSSlots = 4;                 // groups in flight in a workgroup
+constexpr float kPSFirst = -1.f;            // in place of a first row's sigmoid (>= 0 or NaN)
 static_assert(kPSSub * kPSC == 64 * kPSTeam && kGP % kPSSub == 0 && kPSRows < 64 &&
                   kGP < 256 && 2 * kGW <= kGP, "group shape");
 
@@ -1786,29 +1787,46 @@ k_pscan(const int* __restrict__ n_groups, int* __restrict__ ticket, unsigned tag
                     ss[q] = i0 + q < n ? ss[q] : 1.f;
                 }
             }
+            // a cell's first row: its state is vv, whatever came before.  A group
+            // of one cell has it on top, where the state is 0; in a group of
+            // several a product with 0 would let the previous cell's infinity or
+            // NaN through, so the row is marked and its state selected (two more
+            // instructions a row: 200k records at 80 x 64 1.438 -> 1.439 ms, 1.25 M
+            // at 640 x 480 9.23 -> 9.28).
+            const bool multi = (flags & kGMulti) != 0;
             if (flags & kGStart) {
                 const unsigned long long fw = mask_window(S.mfirst, i0);
                 #pragma unroll
                 for (int q = 0; q < kPSRows; ++q)
                     if ((fw >> q) & 1u) {
                         vv[q] = fmaf(ss[q], gload(S.srow[i0 + q] + ch), vv[q]);
-                        ss[q] = 0.f;
+                        ss[q] = multi ? kPSFirst : 0.f;
                     }
             }
             float A = 1.f, B = 0.f;
-            #pragma unroll
-            for (int q = 0; q < kPSRows; ++q) {
-                A *= ss[q];
-                B = fmaf(ss[q], B, vv[q]);
+            if (multi) {
+                // (A is read of row blocks without a first row only)
+                #pragma unroll
+                for (int q = 0; q < kPSRows; ++q) {
+                    A *= ss[q];
+                    B = ss[q] == kPSFirst ? vv[q] : fmaf(ss[q], B, vv[q]);
+                }
+            } else {
+                #pragma unroll
+                for (int q = 0; q < kPSRows; ++q) {
+                    A *= ss[q];
+                    B = fmaf(ss[q], B, vv[q]);
+                }
             }
             sA[g & 1][sub][ch] = A;
             sB[g & 1][sub][ch] = B;
             lds_arrive(&S.mapped);
             lds_wait(&starts, g + 1);
             float h = sA[g & 1][sub][ch];
+            // (one loop for both kinds of group: a second copy spills 29 registers)
             #pragma unroll
             for (int q = 0; q < kPSRows; ++q) {
-                h = fmaf(ss[q], h, vv[q]);
+                h = ss[q] == kPSFirst ? vv[q] : fmaf(ss[q], h, vv[q]);
                 vv[q] = h;
             }
             float* const hb = Hout + __builtin_amdgcn_readfirstlane(S.slab) * kPSC + ch;
@@ -1958,11 +1976,15 @@ k_pscan(const int* __restrict__ n_groups, int* __restrict__ ticket, unsigned tag
             const int word = __builtin_amdgcn_readfirstlane(S.word);
             const int r = __builtin_amdgcn_readfirstlane(S.r);
             const int cc = __builtin_amdgcn_readfirstlane(S.slab) * kPSC + cl;
+            // (of a group of several cells only the start states are used: a row
+            // block that holds a cell's first row ends in a state of its own)
             float a[kPSSub], b[kPSSub], SA = 1.f, SB = 0.f;
+            bool own[kPSSub] = {};
             #pragma unroll
             for (int q = 0; q < kPSSub; ++q) {
                 a[q] = sA[g & 1][q][cl];
                 b[q] = sB[g & 1][q][cl];
+                if (flags & kGMulti) own[q] = mask_window(S.mfirst, q * kPSRows) != 0;
             }
             #pragma unroll
             for (int q = 0; q < kPSSub; ++q) {
@@ -1985,7 +2007,7 @@ k_pscan(const int* __restrict__ n_groups, int* __restrict__ ticket, unsigned tag
             #pragma unroll
             for (int q = 0; q < kPSSub; ++q) {
                 if (con) sA[g & 1][q][cl] = h;
-                h = fmaf(a[q], h, b[q]);
+                h = own[q] ? b[q] : fmaf(a[q], h, b[q]);
             }
             lds_arrive(&starts);
         }
