@@ -1576,7 +1576,8 @@ struct PsSlot {
     float* srow[kGP];               // state row of a pair's cell (groups with a cell end)
     unsigned long long mfirst[kPSMask], mlast[kPSMask], mneed[kPSMask];
     int ids[kGP];                   // 9 record + delta
-    unsigned char tsl[kPSTiles * 16], tdel[kPSTiles];   // pairs and delta of each tile
+    alignas(4) unsigned char tsl[kPSTiles * 16];        // pairs of each tile
+    unsigned char tdel[kPSTiles];                       // its delta
     int ntiles, n, flags, word, r, slab;
     int taken;                      // tiles taken
     // arrivals over all groups that had the slot (a wave reaches the slot's next
@@ -1896,7 +1897,7 @@ k_pscan(const int* __restrict__ n_groups, int* __restrict__ ticket, unsigned tag
             const int slab = NS == 1 ? 0 : tk % NS;
             if (lane < kPatch) dcnt[lane] = 0;
             for (int i = lane; i < kPSTiles * 16 / 4; i += 64)
-                reinterpret_cast<int*>(S.tsl)[i] = kGP * 0x01010101;
+                reinterpret_cast<uint32_t*>(S.tsl)[i] = kGP * 0x01010101u;
             int rank[kPSMask], delta[kPSMask];
             #pragma unroll
             for (int j = 0; j < kPSMask; ++j) {
