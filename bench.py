@@ -622,13 +622,15 @@ def batch_bench(a, d, recs, n, S, steps, warmup, desc, tmp) -> int:
 TRAFFIC_PHASES = {
     "k_pscan<24, 48>": ["L4.proj"], "k_pscan<48, 48>": ["L5.proj"], "k_pscan<48, 96>": ["L6.proj"],
     "k_pscan<96, 96>": ["L7.proj"],
-    "k_outt<24, 48, 2, 1>": ["L4.out"], "k_outt<48, 48, 1, 3>": ["L5.out"],
-    "k_outt<48, 96, 1, 3>": ["L6.out"], "k_outt<96, 96, 1, 3>": ["L7.out"],
+    "k_outt<24, 48>": ["L4.out"], "k_outt<48, 48>": ["L5.out"], "k_outt<48, 96>": ["L6.out"],
+    "k_outt<96, 96>": ["L7.out"],
     "k_head": ["head"], "k_head_linear": ["head"], "k_emit": ["emit"],
 }
 ORDER_KERNELS = ("k_decode", "k_small_order", "k_rs_hist", "k_exscan", "k_rs_scatter", "k_runs", "k_keys2",
                  "k_keyscan", "k_s2_tables", "k_pair_rank", "k_key_groups", "k_keys3a", "k_place3",
                  "k_tdrop3", "k_keys3b", "k_group_order")
+# one launch of either per call (the second for calls of few records and cells)
+CALL_KERNELS = ("k_decode", "k_small_order")
 
 
 def _traffic_key(k: str):
@@ -665,16 +667,18 @@ def pmc_summary(fetch_dir, write_dir, cfetch_dir, cwrite_dir, copy_bytes, comman
 
     def per_phase(rs):
         seen, out = collections.Counter(), collections.defaultdict(float)
-        calls = sum(1 for r in rs if _kname(r["Kernel_Name"]) == "k_decode")
+        calls = sum(1 for r in rs if _kname(r["Kernel_Name"]).split("<")[0] in CALL_KERNELS)
+        if not calls:
+            raise ValueError("no whole-ring drain call in the counter files")
         for r in rs:
             k = _kname(r["Kernel_Name"])
             v = float(r["Counter_Value"]) * 1024.0
             key = _traffic_key(k)
             if k.split("<")[0] in ORDER_KERNELS:
-                out["order"] += v / max(1, calls)
+                out["order"] += v / calls
             elif key is not None:
                 ph = TRAFFIC_PHASES[key]
-                out[ph[seen[key] % len(ph)]] += v / max(1, calls)
+                out[ph[seen[key] % len(ph)]] += v / calls
                 seen[key] += 1
         return out
 
