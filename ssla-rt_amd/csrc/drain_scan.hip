@@ -2942,73 +2942,73 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
             hipLaunchKernelGGL(k_small_order<false>, grid, dim3(kScanThreads), 0, st, E, tab, w.bd, G,
                                w.X0, o, psrc, w.packed, npk);
     } else {
-    // ---- decode (and the fills); stable radix sort of the records by s2 key --
-    {
-        const int ndec = (int)grid1(E, kDecRec), fblk = (int)grid1(std::max<int>(std::max<int>((int)nk2, 16), nv), 256);
-        const int npk = (int)((PackLayout<true>::off[8] + 255) / 256);
-        hipLaunchKernelGGL(k_decode, dim3(ndec + fblk * kFills + npk + 1), dim3(256), 0, st, E, tab,
-                           w.bd, G, w.X0, w.cell2, w.owner, w.ka, w.va, ndec, f, fblk, psrc,
-                           w.packed, npk);
-    }
-    const int bits2 = bits_for(nk2);
-    const int passes = (bits2 + kRMaxBits - 1) / kRMaxBits;
-    const int T = (int)grid1(E, kRTile);
-    uint32_t *kin = w.ka, *vin = nullptr, *kout = w.kb, *vout = w.vb;
-    for (int ps = 0, shift = 0; ps < passes; ++ps) {
-        const int bits = (bits2 - shift + (passes - ps) - 1) / (passes - ps);
-        if ((1 << bits) * T > w.bh_ints) {
-            set_error("drain: radix histogram larger than its workspace");
-            return SSLA_ERR_STATE;
+        // ---- decode (and the fills); stable radix sort of the records by s2 key --
+        {
+            const int ndec = (int)grid1(E, kDecRec), fblk = (int)grid1(std::max<int>(std::max<int>((int)nk2, 16), nv), 256);
+            const int npk = (int)((PackLayout<true>::off[8] + 255) / 256);
+            hipLaunchKernelGGL(k_decode, dim3(ndec + fblk * kFills + npk + 1), dim3(256), 0, st, E, tab,
+                               w.bd, G, w.X0, w.cell2, w.owner, w.ka, w.va, ndec, f, fblk, psrc,
+                               w.packed, npk);
         }
-        // a one-pass sort's digit is the whole key: bins for the keys present
-        // (nk2 values and the keyless records' nk2) only
-        const int nbins = passes == 1 ? (int)nk2 + 1 : 1 << bits;
-        hipLaunchKernelGGL(k_rs_hist, dim3(T), dim3(kRThreads), 0, st, E, kin, shift, bits, nbins,
-                           T, w.bh);
-        hipLaunchKernelGGL(k_exscan, dim3(1), dim3(kScanThreads), 0, st, nbins * T, w.bh);
-        hipLaunchKernelGGL(k_rs_scatter, dim3(T), dim3(kRThreads), 0, st, E, kin, vin, kout, vout,
-                           ps == passes - 1 ? w.sidx : nullptr, shift, bits, nbins, T, w.bh);
-        shift += bits;
-        // the next pass writes the pair of buffers this pass read from
-        uint32_t* const k2 = kout == w.kb ? w.ka : w.kb;
-        uint32_t* const v2 = vout == w.vb ? w.va : w.vb;
-        kin = kout;
-        vin = vout;
-        kout = k2;
-        vout = v2;
-    }
-    // the sorted s2 order, and the buffers the s3 order is placed in
-    K2 = kin;
-    V2 = vin;
-    K3 = kout;
-    V3 = vout;
-    // ---- counters, tdrop_s2, the pass-2 list, s2 pair and group tables -----
-    if (passes == 1 && nk2 <= (uint32_t)kScanThreads) {
-        // the one pass's histogram holds the run bounds: the key tables and
-        // their scans in one workgroup
-        const KeyHist kh{G.C2, G.W2, G.H2, T, G.window, (const int*)w.bh, w.st2, w.en2, w.bd,
-                         w.old2};
-        if (gt2)
-            hipLaunchKernelGGL((k_keyscan<true, true>), dim3(1), dim3(kScanThreads), 0, st, (int)nk2,
-                               (const int*)nullptr, w.pst2, (int*)nullptr, w.goff2, w.n2, w.off2,
-                               w.counts + 0, kh, GroupTab{nv, w.glist, w.counts + 6});
-        else
-            hipLaunchKernelGGL((k_keyscan<true, false>), dim3(1), dim3(kScanThreads), 0, st, (int)nk2,
-                               (const int*)nullptr, w.pst2, (int*)nullptr, w.goff2, w.n2, w.off2,
-                               w.counts + 0, kh, GroupTab{});
-    } else {
-        hipLaunchKernelGGL(k_runs, dim3(grid1(E, 256)), dim3(256), 0, st, E, K2, nk2, w.st2, w.en2);
-        hipLaunchKernelGGL(k_keys2, dim3(grid1(nk2, 256)), dim3(256), 0, st, nk2, G.C2, G.W2, G.H2,
-                           w.st2, w.en2, w.bd, G.window, w.old2, w.n2, w.pcnt);
-        if (gt2)
-            hipLaunchKernelGGL((k_keyscan<false, true>), dim3(1), dim3(kScanThreads), 0, st, (int)nk2,
-                               w.pcnt, w.pst2, (int*)nullptr, w.goff2, w.n2, w.off2, w.counts + 0,
-                               KeyHist{}, GroupTab{nv, w.glist, w.counts + 6});
-        else
-            hipLaunchKernelGGL((k_keyscan<false, false>), dim3(1), dim3(kScanThreads), 0, st, (int)nk2,
-                               w.pcnt, w.pst2, (int*)nullptr, w.goff2, w.n2, w.off2, w.counts + 0,
-                               KeyHist{}, GroupTab{});
-    }
+        const int bits2 = bits_for(nk2);
+        const int passes = (bits2 + kRMaxBits - 1) / kRMaxBits;
+        const int T = (int)grid1(E, kRTile);
+        uint32_t *kin = w.ka, *vin = nullptr, *kout = w.kb, *vout = w.vb;
+        for (int ps = 0, shift = 0; ps < passes; ++ps) {
+            const int bits = (bits2 - shift + (passes - ps) - 1) / (passes - ps);
+            if ((1 << bits) * T > w.bh_ints) {
+                set_error("drain: radix histogram larger than its workspace");
+                return SSLA_ERR_STATE;
+            }
+            // a one-pass sort's digit is the whole key: bins for the keys present
+            // (nk2 values and the keyless records' nk2) only
+            const int nbins = passes == 1 ? (int)nk2 + 1 : 1 << bits;
+            hipLaunchKernelGGL(k_rs_hist, dim3(T), dim3(kRThreads), 0, st, E, kin, shift, bits, nbins,
+                               T, w.bh);
+            hipLaunchKernelGGL(k_exscan, dim3(1), dim3(kScanThreads), 0, st, nbins * T, w.bh);
+            hipLaunchKernelGGL(k_rs_scatter, dim3(T), dim3(kRThreads), 0, st, E, kin, vin, kout, vout,
+                               ps == passes - 1 ? w.sidx : nullptr, shift, bits, nbins, T, w.bh);
+            shift += bits;
+            // the next pass writes the pair of buffers this pass read from
+            uint32_t* const k2 = kout == w.kb ? w.ka : w.kb;
+            uint32_t* const v2 = vout == w.vb ? w.va : w.vb;
+            kin = kout;
+            vin = vout;
+            kout = k2;
+            vout = v2;
+        }
+        // the sorted s2 order, and the buffers the s3 order is placed in
+        K2 = kin;
+        V2 = vin;
+        K3 = kout;
+        V3 = vout;
+        // ---- counters, tdrop_s2, the pass-2 list, s2 pair and group tables -----
+        if (passes == 1 && nk2 <= (uint32_t)kScanThreads) {
+            // the one pass's histogram holds the run bounds: the key tables and
+            // their scans in one workgroup
+            const KeyHist kh{G.C2, G.W2, G.H2, T, G.window, (const int*)w.bh, w.st2, w.en2, w.bd,
+                             w.old2};
+            if (gt2)
+                hipLaunchKernelGGL((k_keyscan<true, true>), dim3(1), dim3(kScanThreads), 0, st, (int)nk2,
+                                   (const int*)nullptr, w.pst2, (int*)nullptr, w.goff2, w.n2, w.off2,
+                                   w.counts + 0, kh, GroupTab{nv, w.glist, w.counts + 6});
+            else
+                hipLaunchKernelGGL((k_keyscan<true, false>), dim3(1), dim3(kScanThreads), 0, st, (int)nk2,
+                                   (const int*)nullptr, w.pst2, (int*)nullptr, w.goff2, w.n2, w.off2,
+                                   w.counts + 0, kh, GroupTab{});
+        } else {
+            hipLaunchKernelGGL(k_runs, dim3(grid1(E, 256)), dim3(256), 0, st, E, K2, nk2, w.st2, w.en2);
+            hipLaunchKernelGGL(k_keys2, dim3(grid1(nk2, 256)), dim3(256), 0, st, nk2, G.C2, G.W2, G.H2,
+                               w.st2, w.en2, w.bd, G.window, w.old2, w.n2, w.pcnt);
+            if (gt2)
+                hipLaunchKernelGGL((k_keyscan<false, true>), dim3(1), dim3(kScanThreads), 0, st, (int)nk2,
+                                   w.pcnt, w.pst2, (int*)nullptr, w.goff2, w.n2, w.off2, w.counts + 0,
+                                   KeyHist{}, GroupTab{nv, w.glist, w.counts + 6});
+            else
+                hipLaunchKernelGGL((k_keyscan<false, false>), dim3(1), dim3(kScanThreads), 0, st, (int)nk2,
+                                   w.pcnt, w.pst2, (int*)nullptr, w.goff2, w.n2, w.off2, w.counts + 0,
+                                   KeyHist{}, GroupTab{});
+        }
     }
     if (!small_all) {
         const unsigned nbr = grid1(E, 256);
@@ -3023,15 +3023,15 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
             hipLaunchKernelGGL(k_group_order, dim3(1), dim3(kScanThreads), 0, st, (int)nk2, nv, w.pst2,
                                w.goff2, w.gcnt, w.gend, w.ghist, w.gw, w.gstart, w.gbase, w.glist,
                                w.counts + 6);
-    // The s3 ordering needs only the s2 order, pass2 and the old counters, so
-    // it runs on the side stream while L4 and L5 run here; L6 waits for it.
-    // Its launches are sized by E; the pass-2 count stays on the device.  Its
-    // event sits before L4's projection, so the side stream's small kernels
-    // start beside the projection rather than beside the latency-bound parts
-    // that follow it.
-    HIPCHK(hipEventRecord(w.s2_ordered, st));
-    end.side = true;
-    HIPCHK(hipStreamWaitEvent(s3, w.s2_ordered, 0));
+        // The s3 ordering needs only the s2 order, pass2 and the old counters, so
+        // it runs on the side stream while L4 and L5 run here; L6 waits for it.
+        // Its launches are sized by E; the pass-2 count stays on the device.  Its
+        // event sits before L4's projection, so the side stream's small kernels
+        // start beside the projection rather than beside the latency-bound parts
+        // that follow it.
+        HIPCHK(hipEventRecord(w.s2_ordered, st));
+        end.side = true;
+        HIPCHK(hipStreamWaitEvent(s3, w.s2_ordered, 0));
     }
     MARK();
     // The pass-2 and pass-3 counts stay on the device; the launches over their
@@ -3081,7 +3081,7 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
     do {                                                                                            \
         if (few(N))                                                                                 \
             hipLaunchKernelGGL((k_outt<IN, OUT, 1, KSF>), dim3(grid1(N, 16)),                        \
-                               dim3(64 * KSF), 0, st,       E, COUNT, LIST, XIN, w.cell2, SH, G.W2,  \
+                               dim3(64 * KSF), 0, st, E, COUNT, LIST, XIN, w.cell2, SH, G.W2,  \
                                WL, HL, w.HR, pk.po[LI], L[LI].ln_gamma, L[LI].ln_beta, XOUT);       \
         else                                                                                        \
             hipLaunchKernelGGL((k_outt<IN, OUT, RT, KS, WPS>), dim3(grid1(N, 16 * RT)), dim3(64 * KS), \
@@ -3095,40 +3095,40 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
     // (enqueued after L4's launches: the host needs a few microseconds per
     // launch, and L4 keeps the device busy meanwhile)
     if (!small_all) {
-    hipLaunchKernelGGL(k_keys3a, dim3(grid1(nk3, 256)), dim3(256), 0, s3, nk3, G, w.n2, w.bd,
-                       w.t3, w.n3);
-    hipLaunchKernelGGL((k_keyscan<false, false>), dim3(1), dim3(kScanThreads), 0, s3, (int)nk3, w.t3,
-                       w.st3, w.en3, (int*)nullptr, w.n3, w.off3, w.counts + 1, KeyHist{},
-                       GroupTab{});
-    hipLaunchKernelGGL(k_place3, dim3(grid1(nmax2, 256)), dim3(256), 0, s3, (const int*)(w.counts + 0),
-                       w.list2, w.bd, G, w.cell2, w.sidx, V2, w.st2, w.en2, w.old2, w.st3, K3, V3,
-                       w.key3g);
-    hipLaunchKernelGGL(k_tdrop3, dim3(grid1(nmax2, 256)), dim3(256), 0, s3, (const int*)(w.counts + 0),
-                       K3, V3, nk3, G.C3, w.st3, w.off3, w.bd, G.window, w.owner,
-                       have_head ? 1 : 0, w.pass3, w.list3, w.last3, w.cnt3);
-    hipLaunchKernelGGL(k_keys3b, dim3(grid1(nk3, 256)), dim3(256), 0, s3, nk3, G, w.t3, w.bd,
-                       w.pcnt);
-    if (gt3) {
-        hipLaunchKernelGGL((k_keyscan<false, true>), dim3(1), dim3(kScanThreads), 0, s3, (int)nk3,
-                           w.pcnt, w.pst3, (int*)nullptr, w.goff3, (const int*)nullptr, (int*)nullptr,
-                           (int*)nullptr, KeyHist{}, GroupTab{nv, w.glist3, w.counts + 7});
-    } else {
-        hipLaunchKernelGGL((k_keyscan<false, false>), dim3(1), dim3(kScanThreads), 0, s3, (int)nk3,
-                           w.pcnt, w.pst3, (int*)nullptr, w.goff3, (const int*)nullptr, (int*)nullptr,
-                           (int*)nullptr, KeyHist{}, GroupTab{});
-        hipLaunchKernelGGL(k_key_groups, dim3(grid1(nk3, 256)), dim3(256), 0, s3, nk3, w.pst3, w.gcnt3,
-                           w.gend3, w.ghist3, w.gw3);
-        hipLaunchKernelGGL(k_group_order, dim3(1), dim3(kScanThreads), 0, s3, (int)nk3, nv, w.pst3,
-                           w.goff3, w.gcnt3, w.gend3, w.ghist3, w.gw3, w.gstart3, w.gbase3, w.glist3,
-                           w.counts + 7);
-    }
+        hipLaunchKernelGGL(k_keys3a, dim3(grid1(nk3, 256)), dim3(256), 0, s3, nk3, G, w.n2, w.bd,
+                           w.t3, w.n3);
+        hipLaunchKernelGGL((k_keyscan<false, false>), dim3(1), dim3(kScanThreads), 0, s3, (int)nk3, w.t3,
+                           w.st3, w.en3, (int*)nullptr, w.n3, w.off3, w.counts + 1, KeyHist{},
+                           GroupTab{});
+        hipLaunchKernelGGL(k_place3, dim3(grid1(nmax2, 256)), dim3(256), 0, s3, (const int*)(w.counts + 0),
+                           w.list2, w.bd, G, w.cell2, w.sidx, V2, w.st2, w.en2, w.old2, w.st3, K3, V3,
+                           w.key3g);
+        hipLaunchKernelGGL(k_tdrop3, dim3(grid1(nmax2, 256)), dim3(256), 0, s3, (const int*)(w.counts + 0),
+                           K3, V3, nk3, G.C3, w.st3, w.off3, w.bd, G.window, w.owner,
+                           have_head ? 1 : 0, w.pass3, w.list3, w.last3, w.cnt3);
+        hipLaunchKernelGGL(k_keys3b, dim3(grid1(nk3, 256)), dim3(256), 0, s3, nk3, G, w.t3, w.bd,
+                           w.pcnt);
+        if (gt3) {
+            hipLaunchKernelGGL((k_keyscan<false, true>), dim3(1), dim3(kScanThreads), 0, s3, (int)nk3,
+                               w.pcnt, w.pst3, (int*)nullptr, w.goff3, (const int*)nullptr, (int*)nullptr,
+                               (int*)nullptr, KeyHist{}, GroupTab{nv, w.glist3, w.counts + 7});
+        } else {
+            hipLaunchKernelGGL((k_keyscan<false, false>), dim3(1), dim3(kScanThreads), 0, s3, (int)nk3,
+                               w.pcnt, w.pst3, (int*)nullptr, w.goff3, (const int*)nullptr, (int*)nullptr,
+                               (int*)nullptr, KeyHist{}, GroupTab{});
+            hipLaunchKernelGGL(k_key_groups, dim3(grid1(nk3, 256)), dim3(256), 0, s3, nk3, w.pst3, w.gcnt3,
+                               w.gend3, w.ghist3, w.gw3);
+            hipLaunchKernelGGL(k_group_order, dim3(1), dim3(kScanThreads), 0, s3, (int)nk3, nv, w.pst3,
+                               w.goff3, w.gcnt3, w.gend3, w.ghist3, w.gw3, w.gstart3, w.gbase3, w.glist3,
+                               w.counts + 7);
+        }
 #define PAIR_RANK3(SMALL)                                                                             \
     hipLaunchKernelGGL(k_pair_rank<SMALL>, dim3(grid1(nmax2, 256)), dim3(256), 0, s3, E, n2_dev, K3, V3, nk3, \
                        G.C3, G.W3, G.H3, w.st3, w.en3, w.pst3, w.pent3, w.pass3)
-    if (nmax2 <= kSmallRec) PAIR_RANK3(true);
-    else PAIR_RANK3(false);
+        if (nmax2 <= kSmallRec) PAIR_RANK3(true);
+        else PAIR_RANK3(false);
 #undef PAIR_RANK3
-    HIPCHK(hipEventRecord(w.s3_ordered, s3));
+        HIPCHK(hipEventRecord(w.s3_ordered, s3));
     }
     HIPCHK(hipGetLastError());
     // ---- L5: 48 -> 48, state for all records, output for pass2 ---------------
