@@ -470,15 +470,16 @@ def _roofline_phase(per):
     return max(single, key=single.get)
 
 
-def _roofline(per, flops, byts, iface, dom):
+def _roofline(per, flops, byts, iface, dom, profiled):
+    """profiled: the call is the one the committed rocprofv3 summaries are of."""
     kname = PHASE_KERNEL.get(dom, dom)
-    traffic = hbm_traffic(dom)
+    traffic = hbm_traffic(dom) if profiled else None
     fl, by, ib = flops.get(dom, 0.0), byts.get(dom, 0.0), iface.get(dom, 0.0)
     base = {"kernel": f"{kname} ({dom})", "traffic": traffic, "avg_launch_ms": round(per[dom], 5),
             "algorithmic_bytes_per_launch": int(by), "algorithmic_flops_per_launch": int(fl),
             "interface_bytes_per_launch": int(ib),
             "interface_gbs": round(ib / (per[dom] * 1e-3) / 1e9, 1)}
-    tr = trace_ms(dom)
+    tr = trace_ms(dom) if profiled else None
     if by > 0 and fl / by < RIDGE:
         ach = by / (per[dom] * 1e-3) / 1e9
         r = dict(base, bound="hbm", achieved=round(ach, 2), peak=PEAK_HBM_GBS, unit="GB/s",
@@ -946,9 +947,8 @@ def main() -> int:
                 dst[k] = dst.get(k, 0.0) + v
         total_mac += m_
     flops, byts, ibyts = launch_work(flops, byts, ibyts)
-    roof = _roofline(per_timed, flops, byts, ibyts, roof_phase)
-    if a.workload != "80x64":
-        roof["traffic"] = None           # the committed PMC summary is of the 80x64 workload
+    profiled = a.workload == "80x64" and n == wl["n"]
+    roof = _roofline(per_timed, flops, byts, ibyts, roof_phase, profiled)
     if roof.get("unit") == "GB/s":
         # what this device reaches on write-dominated traffic (the published
         # 8 TB/s counts read and write capacity together)
@@ -970,7 +970,7 @@ def main() -> int:
     whole = 2.0 * total_mac / (ms_step * 1e-3) / 1e12
     iface = sum(ibyts.values())
     comp = sum(compulsory_bytes(r.x, r.y, o["pass2"], H2, W2) for r, o in zip(recs, outs))
-    measured = hbm_traffic() if a.workload == "80x64" else None
+    measured = hbm_traffic() if profiled else None
     res = {
         "metric": METRIC, "value": round(value, 3), "unit": "kev/s", "n_gpus": 1,
         "steps": steps, "warmup": warmup, "ms_per_step": round(ms_step, 4),
@@ -983,7 +983,7 @@ def main() -> int:
         "whole_drain_tflops": round(whole, 4),
         # HBM bytes per call: the compulsory ones (records, hidden-state RMW
         # per patch, output slots, counters) against what rocprofv3 measured
-        # for this build (committed PMC summary; 80x64 workload only)
+        # for this build (committed PMC summary; the default call only)
         "compulsory_hbm_bytes": int(comp),
         "measured_hbm_bytes": measured,
         "measured_over_compulsory": round(measured / comp, 3) if measured else None,
@@ -1004,7 +1004,7 @@ def main() -> int:
                                   "(h rows)",
         "roofline_by_phase": {
             k: {x: r[x] for x in ("bound", "achieved", "unit", "frac", "interface_gbs")}
-            for k, r in ((k, _roofline(per, flops, byts, ibyts, k)) for k in per
+            for k, r in ((k, _roofline(per, flops, byts, ibyts, k, profiled)) for k in per
                          if k not in ("order", "head") and per[k] > 0
                          and (flops.get(k, 0.0) > 0 or byts.get(k, 0.0) > 0))},
     }

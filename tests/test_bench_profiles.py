@@ -49,3 +49,15 @@ def test_no_call_is_an_error(tmp_path):
     copy = _counters(tmp_path / "c", ["copy"], 1, 8)
     with pytest.raises(ValueError, match="no whole-ring drain"):
         bench.pmc_summary(fetch, fetch, copy, copy, 8 * 1024, "cmd")
+
+
+def test_committed_profiles_are_of_the_default_call_only():
+    """The committed traffic and trace are of 200,000 records at 80x64: no
+    other call's roofline line takes its traffic or launch time from them."""
+    per, flops, byts, iface = {"L5.proj": 1.9}, {"L5.proj": 1e11}, {"L5.proj": 4e9}, {"L5.proj": 8e8}
+    own = bench._roofline(per, flops, byts, iface, "L5.proj", True)
+    assert own["traffic"] and own["avg_launch_ms_kernel_trace"] and "frac_kernel_trace" in own
+    other = bench._roofline(per, flops, byts, iface, "L5.proj", False)
+    assert other["traffic"] is None
+    assert "frac_kernel_trace" not in other and "avg_launch_ms_kernel_trace" not in other
+    assert other["frac"] == own["frac"]
