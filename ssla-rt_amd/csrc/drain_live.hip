@@ -366,8 +366,11 @@ __device__ __forceinline__ void build_pairs(SL& S, int B, const unsigned char* s
 // flight, the prefetched item included, before each item.)  An item whose delta
 // has no pair skips its products.  MTL: 16-record tiles of the layer's records.
 // Per batch of 8 (16 streams) L4..L7 took 9.9 / 9.6 / 12.9 / 16.4 us with the loop
-// and 7.1 / 9.0 / 10.4 / 13.6 now; the weights at a CU's 64 B a clock would take
-// 0.5 / 1.1 / 2.2 / 4.3.  Five items ahead (L4..L6) were 5% slower.
+// and 7.1 / 9.0 / 10.4 / 13.6 now; the packed weights (166 / 249 / 498 / 995 KB)
+// at a CU's 64 B a clock and 2.4 GHz take 1.1 / 1.6 / 3.2 / 6.5 with the q columns,
+// 0.7 / 1.1 / 2.2 / 4.3 without.  Five items ahead (L4..L6) were 5% slower.  Live at
+// 2 Mev/s, one workgroup for the grid: p50 / p99 274 / 390 -> 220 / 318 us; one for
+// each of eight strips 169 / 270 -> 145 / 233 (phase_out's change included).
 //   A operand: the weights, lane (i, k) = (lane % 16, lane / 16) holds channel i
 //   B operand: the records;  D: lane holds channels 4k..4k+3 of record i, one
 //   float4 of its row

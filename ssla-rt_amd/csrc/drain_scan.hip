@@ -1449,16 +1449,17 @@ k_small_order(int E, BlockTable tab, BlockDesc* __restrict__ bd_out, Geometry G,
 //
 // Bounds and measurements (200k records at 80 x 64, L4 / L5 / L6 / L7): the fp32
 // matrix cores need 67 / 135 / 62 / 127 us for the tiles (11 pairs of a tile's 16
-// are real: 9 deltas share a group's 176 pairs), and were busy 35-52% of 0.20 /
-// 0.28 / 0.155 / 0.235 ms.  The two launches this replaced (projection to pair
-// rows in memory, one-pass scan over them) took 0.41 / 0.38 / 0.22 / 0.26 ms and
-// moved 4 GB more per call; the drain went 1.80 -> 1.40 ms.  Loads are not the
+// are real: 9 deltas share a group's 176 pairs), and are busy 35 / 50 / 42 / 54% of
+// 0.21 / 0.30 / 0.157 / 0.25 ms.  The two launches this replaced (projection to pair
+// rows in memory, one-pass scan over them) took 0.41 / 0.38 / 0.22 / 0.26 ms; a call
+// moved 6.0 GB and moves 2.4, and went from 1.80 to 1.43 ms.  Loads are not the
 // bound (rows or weights from the L1 changed the times by 2-8%).  Measured on the
-// way: workgroups of 6 waves do not pair on a CU (2.05 ms per call); 8 waves that
-// run all phases in turn, two workgroups per CU, 1.70; the same with look-back
-// and replay of a group behind the tiles of the next, 1.52; one row team of 3
-// waves and 11 tile waves, 1.51; two interleaved accumulator chains per tile
-// wave, 1.43 (a single dependent chain forwards its accumulator).
+// way, in ms per call beside 1.40 for the kept form in the same runs: workgroups of
+// 6 waves do not pair on a CU (2.05); 8 waves that run all phases in turn, two
+// workgroups per CU, 1.70; the same with look-back and replay of a group behind the
+// tiles of the next, 1.52; one row team of 3 waves and 11 tile waves, 1.51; two
+// interleaved accumulator chains per tile wave, 1.43 (a single dependent chain
+// forwards its accumulator).
 // ---------------------------------------------------------------------------
 constexpr int kTM = 64;     // records per head workgroup
 
@@ -2440,8 +2441,8 @@ k_head_linear(const int* __restrict__ n_dev, const int* __restrict__ list,
 
 // Output slots (...celled.cuh:1233-1247 conventions) and raw head rows.
 // Output slots (392 B = 49 eight-byte words) and head rows as coalesced
-// 8-byte stores: 32 records per 256-thread workgroup.
-// (a small call: 8, so that its few records are not one workgroup's loop)
+// 8-byte stores: 128 records per 256-thread workgroup (a small call: 8, so that
+// its few records are not one workgroup's loop).
 constexpr int kEmitRec = 128, kEmitRecFew = 8;
 
 template <int RPB>
@@ -3047,10 +3048,10 @@ int scan_drain(const HybridS2S3Config* cfg, const HybridInputRec* const* rings,
     const int* const no_list = nullptr;
     // P + S of layer LI over the groups of level LV (their count in
     // counts[NG], ticket counter counts[8 + LI]): h rows to HR where the pair's
-    // record needs the output (ALL: every pair's).  Two workgroups of k_pscan
-    // fit a CU (LDS), and the grid is what is resident at once, or the groups
-    // the call can have: full groups, a tail per cell of more than kGW pairs
-    // and the shared ones, one per window of kGW.
+    // record needs the output (ALL: every pair's).  One workgroup of k_pscan
+    // fits a CU (155,136 B of LDS, 1024 threads), and the grid is one per CU, or
+    // the groups the call can have if they are fewer: full groups, a tail per cell
+    // of more than kGW pairs and the shared ones, one per window of kGW.
     const unsigned long long wait_ticks = (unsigned long long)std::max(w.clk_khz, 1) * 500ull;
     const unsigned cus = w.cus > 0 ? (unsigned)w.cus : 256u;
     auto group_bound = [](long long recs, long long nk) {
